@@ -80,13 +80,6 @@ def _pow2(rng, lo, hi):
     return 1 << rng.randint(lo.bit_length() - 1, hi.bit_length() - 1)
 
 
-def _large_prime_factor(n):
-    for p in (2, 3, 5, 7, 11, 13):
-        while n % p == 0:
-            n //= p
-    return n > 1
-
-
 def _batch(rng, per, lo, hi):
     """A batch so that the points of the call are log-uniform in [lo, hi]."""
     return max(1, int(_log(rng, lo, hi) / per))
