@@ -143,36 +143,45 @@ static void four_step_tables(int64_t ntot, int sign, TableRef &lo, TableRef &hi)
     };
 }
 
-// In-place FP64 radix-2 FFT (host; plan-time table generation only).
-static void fft_pow2_f64(std::vector<double> &re, std::vector<double> &im, int sign)
+// FP64 forward FFT of a 2,3,5-smooth length (host; plan-time table generation only): Stockham
+// passes of radix 4, 2, 3 and 5 with the roots evaluated once.
+static void fft_smooth_f64(std::vector<double> &re, std::vector<double> &im)
 {
     const size_t n = re.size();
-    for (size_t i = 1, j = 0; i < n; i++) {
-        size_t bit = n >> 1;
-        for (; j & bit; bit >>= 1) j ^= bit;
-        j ^= bit;
-        if (i < j) {
-            std::swap(re[i], re[j]);
-            std::swap(im[i], im[j]);
-        }
+    std::vector<double> wr(n), wi(n), tr(n), ti(n);
+    for (size_t m = 0; m < n; m++) {
+        const long double a = -6.283185307179586476925286766559005768L * (long double)m / (long double)n;
+        wr[m] = (double)cosl(a);
+        wi[m] = (double)sinl(a);
     }
-    for (size_t len = 2; len <= n; len <<= 1) {
-        const long double ang = sign * 6.283185307179586476925286766559005768L / (long double)len;
-        std::vector<double> wr(len / 2), wi(len / 2);
-        for (size_t k = 0; k < len / 2; k++) {
-            wr[k] = (double)cosl(ang * (long double)k);
-            wi[k] = (double)sinl(ang * (long double)k);
-        }
-        for (size_t i = 0; i < n; i += len)
-            for (size_t k = 0; k < len / 2; k++) {
-                const double ur = re[i + k], ui = im[i + k];
-                const double xr = re[i + k + len / 2], xi = im[i + k + len / 2];
-                const double vr = xr * wr[k] - xi * wi[k], vi = xr * wi[k] + xi * wr[k];
-                re[i + k] = ur + vr;
-                im[i + k] = ui + vi;
-                re[i + k + len / 2] = ur - vr;
-                im[i + k + len / 2] = ui - vi;
+    size_t ns = 1;
+    while (ns < n) {
+        const size_t left = n / ns;
+        const size_t R = left % 4 == 0 ? 4 : left % 2 == 0 ? 2 : left % 3 == 0 ? 3 : 5;
+        const size_t nbf = n / R, step = n / (ns * R);
+        for (size_t b = 0; b < nbf; b++) {
+            const size_t k = b % ns, d = (b / ns) * ns * R + k;
+            double vr[5], vi[5];
+            for (size_t r = 0; r < R; r++) {
+                const double xr = re[b + r * nbf], xi = im[b + r * nbf];
+                const size_t m = k * r * step;  // < n
+                vr[r] = xr * wr[m] - xi * wi[m];
+                vi[r] = xr * wi[m] + xi * wr[m];
             }
+            for (size_t q = 0; q < R; q++) {
+                double sr = vr[0], si = vi[0];
+                for (size_t r = 1; r < R; r++) {
+                    const size_t m = (r * q % R) * nbf;
+                    sr += vr[r] * wr[m] - vi[r] * wi[m];
+                    si += vr[r] * wi[m] + vi[r] * wr[m];
+                }
+                tr[d + q * ns] = sr;
+                ti[d + q * ns] = si;
+            }
+        }
+        re.swap(tr);
+        im.swap(ti);
+        ns *= R;
     }
 }
 
@@ -211,7 +220,7 @@ static TableRef bluestein_kernel(int64_t N, int64_t M, int sign)
                 im[(size_t)(M - n)] = ci;
             }
         }
-        fft_pow2_f64(re, im, -1);
+        fft_smooth_f64(re, im);
         std::vector<float2> v((size_t)M);
         for (int64_t k = 0; k < M; k++) {
             v[(size_t)k].x = (float)(re[(size_t)k] / (double)M);
@@ -361,6 +370,17 @@ static int64_t big_leaf_min_rows(const Plan &p)
     if (e && e[0]) return std::atoll(e);
     return p.big_leaf_rows > 0 ? p.big_leaf_rows : 256;
 }
+// One launch for a run of stages where a fused kernel exists; SIP_FFT_FUSE=0 at plan time runs the
+// stages one by one (the comparison path of the tests).
+static bool fusing() { return env_flag("SIP_FFT_FUSE", true); }
+
+// LDS pitch (floats) of a transform of n values padded by one word every 16, odd.
+static int lds_pitch(int64_t n)
+{
+    const int lp = (int)(n - 1 + ((n - 1) >> 4)) + 1;
+    return lp | 1;
+}
+
 constexpr int64_t kFillWorkgroups = 512;  // two workgroups per CU of MI355X (256 CUs)
 
 struct Builder {
@@ -802,6 +822,7 @@ struct Builder {
         if (M > (int64_t(1) << 26))
             throw SipError(AsdSip::ACL_ERROR_API_NOT_SUPPORT, "Bluestein length too large");
         const int64_t rows = count(normalize(in.dims));
+        const size_t first = p.stages.size();
         BufRef w = new_ws((size_t)rows * M * 8);
         Lay wl{w, 1, {{rows, M}}};
         TableRef chirp = bluestein_chirp(N, sign);
@@ -810,6 +831,60 @@ struct Builder {
         add_aux(AUX_BLUE_MUL, wl, wl, M, M, bluestein_kernel(N, M, sign), 1.f, "bluestein kernel");
         axis(M, 1, wl, wl, true);
         add_aux(AUX_BLUE_POST, wl, Lay{out.buf, out.es, out.dims}, N, N, chirp, 1.f, "bluestein post");
+        fuse_bluestein(first, N, sign, in, out);
+    }
+
+    // The stages from `first` to the last one run as one launch of `st`'s kernel.
+    void fuse(size_t first, Stage &&st) { p.fusions.push_back(Fusion{first, p.stages.size() - 1, std::move(st)}); }
+
+    // One-launch Bluestein (kernels/bluestein.h) for every length whose convolution fits an
+    // instance (N <= 16384), any strides; the precision form keeps its matrix-core FFT stages.
+    void fuse_bluestein(size_t first, int64_t N, int sign, const Lay &in, const Lay &out)
+    {
+        const BluesteinInstance *bi = p.precision == PREC_FP32 ? find_bluestein_instance(2 * N - 1) : nullptr;
+        if (!bi || !fusing()) return;
+        bool ok = true;
+        Stage st;
+        st.kind = StageKind::Stockham;
+        st.in = in.buf;
+        st.out = out.buf;
+        st.fused_fn = bi->fn;
+        st.sign = sign;
+        StockhamArgs &a = st.sa;
+        std::memset(&a, 0, sizeof(a));
+        a.tin = to_tile(in, &ok, &st.in_tab);
+        a.tout = to_tile(out, &ok, &st.out_tab);
+        a.nfft = count(normalize(in.dims));
+        if (!ok || a.nfft >= (int64_t(1) << 31)) return;
+        a.tin.vec2 = a.tout.vec2 = 0;
+        a.io_mode = IO_C2C;
+        a.in_len = a.out_len = (int32_t)N;
+        a.in_sep = is_user(in.buf) ? 1 : 0;
+        a.out_sep = is_user(out.buf) ? 1 : 0;
+        a.LP = lds_pitch(bi->M);
+        const int T = bi->T;
+        const int64_t per = (int64_t)a.LP * 4;
+        // Column tiles (lanes walk adjacent transforms) 16 wide, rows about 256 threads; fewer rows per
+        // workgroup until the grid has two workgroups per CU, as for the leaf kernels.
+        a.col_direct = (a.tin.unit_f || a.tout.unit_f) ? 1 : 0;
+        int F = a.col_direct ? 16 : std::max(1, 256 / T);
+        while (F > 1 && (F * T > 1024 || F * per > (a.col_direct ? 160 : 48) * 1024)) F = (F + 1) / 2;
+        if (!a.col_direct)
+            while (F > 1 && ((F + 1) / 2) * T >= 64 && (a.nfft + F - 1) / F < kFillWorkgroups) F = (F + 1) / 2;
+        if (F > a.nfft) F = (int)a.nfft;
+        a.F = F;
+        a.div_F = make_fastdiv((uint32_t)F);
+        std::vector<int> rad(bi->radix, bi->radix + bi->npass);
+        st.tw = pass_twiddles_seq(bi->M, rad, -1);
+        std::reverse(rad.begin(), rad.end());
+        st.tw2 = pass_twiddles_seq(bi->M, rad, 1);
+        st.rtw = bluestein_chirp(N, sign);
+        st.tw4lo = bluestein_kernel(N, bi->M, sign);
+        st.grid = dim3((unsigned)((a.nfft + F - 1) / F));
+        st.block = dim3((unsigned)(F * T));
+        st.lds = (size_t)(F * per);
+        st.note = "bluestein " + std::to_string(N) + " on " + std::to_string(bi->M) + " points";
+        fuse(first, std::move(st));
     }
 
     // Real-to-complex transform of the last axis (n reals -> n/2+1 bins per row).
@@ -891,6 +966,8 @@ struct Builder {
 void plan_build(Plan &p)
 {
     p.stages.clear();
+    p.fusions.clear();
+    p.launches.clear();
     p.ws_offsets.clear();
     p.ws_bytes = 0;
     Builder b(p);
@@ -1038,6 +1115,8 @@ void plan_build_gathered(Plan &p, int type, int64_t n, const std::vector<int64_t
     if (!gathered_supported(type, n))
         throw SipError(AsdSip::ACL_ERROR_API_NOT_SUPPORT, "gathered rows not supported for this type / length");
     p.stages.clear();
+    p.fusions.clear();
+    p.launches.clear();
     p.ws_offsets.clear();
     p.ws_bytes = 0;
     p.fftType = type;
@@ -1082,8 +1161,22 @@ Plan::~Plan()
 
 // ====================================================================== device side
 
+std::vector<Stage *> plan_launches(Plan &p)
+{
+    std::vector<Stage *> r;
+    for (size_t i = 0; i < p.stages.size(); i++) {
+        Fusion *f = nullptr;
+        for (Fusion &c : p.fusions)
+            if (c.first == i) f = &c;
+        r.push_back(f ? &f->stage : &p.stages[i]);
+        if (f) i = f->last;
+    }
+    return r;
+}
+
 static const void *stage_kernel(const Stage &s)
 {
+    if (s.fused_fn) return s.fused_fn;
     if (s.inst2d) return s.sign < 0 ? s.inst2d->fwd : s.inst2d->inv;
     if (s.rc) return s.inst->rc[s.sign < 0 ? 0 : 1];
     if (s.sa.split_lds && s.sa.col_direct) return s.inst->cols[(s.sa.tw4_ntot != 0 ? 2 : 0) + (s.sign < 0 ? 0 : 1)];
@@ -1093,11 +1186,12 @@ static const void *stage_kernel(const Stage &s)
     return s.sign < 0 ? s.inst->fwd : s.inst->inv;
 }
 
-bool plan_launchable(const Plan &p)
+bool plan_launchable(Plan &p)
 {
     // gfx950: at most 1024 threads and 160 KiB of LDS (static + dynamic) per workgroup
     constexpr size_t kLdsPerWorkgroup = 160 * 1024;
-    for (const Stage &s : p.stages) {
+    for (const Stage *sp : plan_launches(p)) {
+        const Stage &s = *sp;
         if (s.kind != StageKind::Stockham) continue;
         hipFuncAttributes attr;
         if (hipFuncGetAttributes(&attr, stage_kernel(s)) != hipSuccess) {
@@ -1171,8 +1265,10 @@ void plan_materialize(Plan &p)
 {
     SIP_HIP_CHECK(hipGetDevice(&p.device));
     plan_mark_streaming(p);
+    p.launches = plan_launches(p);
     if (!p.external_tables.empty()) {
-        for (Stage &s : p.stages) {
+        for (Stage *sp : p.launches) {
+            Stage &s = *sp;
             const int64_t *ti = s.in_tab >= 0 ? p.external_tables[(size_t)s.in_tab] : nullptr;
             const int64_t *to = s.out_tab >= 0 ? p.external_tables[(size_t)s.out_tab] : nullptr;
             if (s.kind == StageKind::Stockham) {
@@ -1193,7 +1289,8 @@ void plan_materialize(Plan &p)
             SIP_HIP_CHECK(hipMemcpy(p.row_tables_dev[i], p.row_tables[i].data(), bytes, hipMemcpyHostToDevice));
         }
     }
-    for (Stage &s : p.stages) {
+    for (Stage *sp : p.launches) {
+        Stage &s = *sp;
         if (s.kind == StageKind::Stockham) {
             if (p.external_tables.empty()) {
                 if (s.in_tab >= 0) s.sa.tin.tab = static_cast<const int64_t *>(p.row_tables_dev[(size_t)s.in_tab]);
@@ -1203,7 +1300,7 @@ void plan_materialize(Plan &p)
             if (s.rtw.used()) s.rtw.dev = coeff_get(s.rtw);
             if (s.tw4lo.used()) {
                 s.tw4lo.dev = coeff_get(s.tw4lo);
-                s.tw4hi.dev = coeff_get(s.tw4hi);
+                if (s.tw4hi.used()) s.tw4hi.dev = coeff_get(s.tw4hi);
             }
             s.sa.tw = static_cast<const float2 *>(s.tw.dev->ptr);
             if (s.tw2.used()) {
@@ -1258,7 +1355,8 @@ void plan_execute_sep(Plan &p, const void *in, const void *in_im, void *out, voi
         if (b.kind == BUF_OUT) return static_cast<float *>(out_im);
         return nullptr;
     };
-    for (Stage &s : p.stages) {
+    for (Stage *sp : p.launches) {
+        Stage &s = *sp;
         void *src = resolve(p, s.in, in, out);
         void *dst = resolve(p, s.out, in, out);
         if (s.kind == StageKind::Stockham) {
@@ -1322,6 +1420,13 @@ std::string plan_describe(const Plan &p)
                << ",\"out_len\":" << s.xa.out_len;
         }
         os << "}";
+    }
+    os << "],\"fused\":[";
+    for (size_t i = 0; i < p.fusions.size(); i++) {
+        const Fusion &f = p.fusions[i];
+        os << (i ? "," : "") << "{\"first\":" << f.first << ",\"last\":" << f.last << ",\"note\":\"" << f.stage.note
+           << "\",\"F\":" << f.stage.sa.F << ",\"grid\":" << f.stage.grid.x << ",\"block\":" << f.stage.block.x
+           << ",\"lds\":" << f.stage.lds << "}";
     }
     os << "]}";
     return os.str();

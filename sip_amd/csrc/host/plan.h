@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "../kernels/aux_args.h"
+#include "../kernels/fused_args.h"
 #include "../kernels/stockham_args.h"
 #include "common.h"
 
@@ -89,7 +90,16 @@ struct Stage {
     // Aux
     AuxArgs xa{};
     TableRef tab0;
+    // Kernel of a launch that stands for several stages (Plan::fusions); null for a stage of its own
+    const void *fused_fn = nullptr;
     std::string note;
+};
+
+// Stages first .. last of a plan run as the one launch `stage`. The stage list itself (and so the
+// workspace a caller binds) is the same with and without the fused launch.
+struct Fusion {
+    size_t first = 0, last = 0;
+    Stage stage;
 };
 
 struct Plan {
@@ -106,6 +116,8 @@ struct Plan {
     int device = 0;
 
     std::vector<Stage> stages;
+    std::vector<Fusion> fusions;
+    std::vector<Stage *> launches;  // plan_launches(*this), set by plan_materialize
     std::vector<size_t> ws_offsets;  // byte offset of each workspace region
     size_t ws_bytes = 0;
 
@@ -158,7 +170,9 @@ void plan_materialize(Plan &p);
 void plan_mark_streaming(Plan &p);
 // True when every stage's launch shape (threads, static + dynamic LDS) is within what the device
 // accepts for its kernel; checked before a tuning candidate is materialized or launched.
-bool plan_launchable(const Plan &p);
+bool plan_launchable(Plan &p);
+// What an exec launches, in order: the stages, with each fused run replaced by its one launch.
+std::vector<Stage *> plan_launches(Plan &p);
 // Enqueues the stages on p.stream. in/out are device addresses of the user tensors.
 void plan_execute(Plan &p, const void *in, void *out);
 // Split-plane (C2C_SEP) execution: user buffers are real / imaginary float planes.
@@ -174,6 +188,8 @@ const StockhamInstance *find_instance(int64_t L);
 const StockhamInstance *find_mfma_instance(int64_t L, int mode);
 // Fused 2D tile instance for X x Y slices (X, Y in 32, 64, 128), or null.
 const Stockham2dInstance *find_2d_instance(int64_t X, int64_t Y);
+// One-launch Bluestein instance of the shortest convolution of at least `min_m` points, or null.
+const BluesteinInstance *find_bluestein_instance(int64_t min_m);
 TableRef mfma_dft_table(int mode, int sign);
 // Operand table of the single-plane K = 32 matrix passes (kernels/mfma_split.h).
 TableRef mfma2_dft_table(int mode, int sign);

@@ -52,4 +52,14 @@ const Stockham2dInstance *find_2d_instance(int64_t X, int64_t Y)
     return nullptr;
 }
 
+extern const BluesteinInstance g_bluestein[];
+extern const int g_bluestein_count;
+
+const BluesteinInstance *find_bluestein_instance(int64_t min_m)
+{
+    for (int i = 0; i < g_bluestein_count; i++)  // ascending M
+        if (g_bluestein[i].M >= min_m) return &g_bluestein[i];
+    return nullptr;
+}
+
 }  // namespace sip

@@ -746,8 +746,8 @@ private:
     void keep_resident(const Plan &plan)
     {
         const uint64_t now = ++resident_clock_;
-        for (const Stage &st : plan.stages)
-            for (const TableRef *t : {&st.tw, &st.rtw, &st.tw4lo, &st.tw4hi, &st.mfw, &st.tab0, &st.tw2}) {
+        for (const Stage *st : plan.launches)
+            for (const TableRef *t : {&st->tw, &st->rtw, &st->tw4lo, &st->tw4hi, &st->mfw, &st->tab0, &st->tw2}) {
                 if (!t->dev) continue;
                 auto ins = resident_.emplace(t->dev.get(), Resident{t->dev, now});
                 if (ins.second)
