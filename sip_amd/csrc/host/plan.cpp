@@ -887,6 +887,56 @@ struct Builder {
         fuse(first, std::move(st));
     }
 
+    // One-launch inverse short-time transform (kernels/istft.h): 2,3,5-smooth frame lengths whose
+    // tile of F frames ends the samples of at least half of them (F / 2 <= keep). Shorter hops read
+    // every frame more than twice and keep the staged form, except above 1024 points, where the
+    // staged form splits the frames' transforms in two (1152, hop 144: 215 us): a quarter there.
+    void fuse_istft(size_t first)
+    {
+        const Plan::Istft &q = p.istft;
+        const IstftInstance *ii = p.precision == PREC_FP32 ? find_istft_instance(q.nfft) : nullptr;
+        if (!ii || !fusing()) return;
+        Stage st;
+        st.kind = StageKind::Istft;
+        st.in.kind = BUF_IN;
+        st.out.kind = BUF_OUT;
+        st.fused_fn = ii->fn;
+        st.sign = 1;
+        IstftArgs &a = st.ia;
+        a.frames = q.frames;
+        a.hop = q.hop;
+        a.out_len = q.out_len;
+        a.start = q.nfft / 2;
+        a.halo = (int32_t)((q.nfft + q.hop - 1) / q.hop - 1);
+        a.LP = lds_pitch(ii->L);
+        // as many frames as 1024 threads and half of the LDS hold (two workgroups per CU), in whole
+        // runs of 16 (128-byte loads), at most 64
+        int F = std::min(64, 1024 / ii->T);
+        while (F > 1 && (int64_t)F * a.LP * 4 > 80 * 1024) F--;
+        if (F >= 16) F &= ~15;
+        const int64_t least = q.nfft <= kColumnLeafMax ? 2 : 4;
+        if (least * (F - a.halo) < F) return;
+        // few frames: smaller tiles until every CU has one (640, hop 320, 4 x 103 frames: 21 us on 16
+        // tiles of 32 frames)
+        while (F >= 16 && least * (F / 2 - a.halo) >= F / 2 && q.channel * q.frames < 256 * (int64_t)(F - a.halo))
+            F /= 2;
+        a.F = F;
+        a.keep = F - a.halo;
+        // samples start .. start + out_len - 1 of the span, keep * hop of them per tile
+        a.tiles = (a.start + a.out_len + a.keep * a.hop - 1) / (a.keep * a.hop);
+        const int64_t grid = a.tiles * q.channel;
+        if (grid >= (int64_t(1) << 31) || q.hop >= (int64_t(1) << 20)) return;
+        a.div_F = make_fastdiv((uint32_t)F);
+        a.div_tiles = make_fastdiv((uint32_t)a.tiles);
+        a.div_hop = make_fastdiv((uint32_t)a.hop);
+        st.tw = pass_twiddles_seq(ii->L, std::vector<int>(ii->radix, ii->radix + ii->npass), 1);
+        st.grid = dim3((unsigned)grid);
+        st.block = dim3((unsigned)(F * ii->T));
+        st.lds = (size_t)F * a.LP * 4;
+        st.note = "istft " + std::to_string(q.nfft) + ", hop " + std::to_string(q.hop);
+        fuse(first, std::move(st));
+    }
+
     // Real-to-complex transform of the last axis (n reals -> n/2+1 bins per row).
     void r2c_axis(int64_t n, int sign, int64_t rows, const BufRef &src, const BufRef &dst)
     {
@@ -995,6 +1045,7 @@ void plan_build(Plan &p)
         x.hop = q.hop;
         x.frames = q.frames;
         x.start = q.nfft / 2;
+        b.fuse_istft(0);
         return;
     }
     if (nd == 1) {
@@ -1291,7 +1342,12 @@ void plan_materialize(Plan &p)
     }
     for (Stage *sp : p.launches) {
         Stage &s = *sp;
-        if (s.kind == StageKind::Stockham) {
+        if (s.kind == StageKind::Istft) {
+            s.tw.dev = coeff_get(s.tw);
+            s.ia.tw = static_cast<const float2 *>(s.tw.dev->ptr);
+            if (s.lds > 64 * 1024)
+                SIP_HIP_CHECK(hipFuncSetAttribute(s.fused_fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)s.lds));
+        } else if (s.kind == StageKind::Stockham) {
             if (p.external_tables.empty()) {
                 if (s.in_tab >= 0) s.sa.tin.tab = static_cast<const int64_t *>(p.row_tables_dev[(size_t)s.in_tab]);
                 if (s.out_tab >= 0) s.sa.tout.tab = static_cast<const int64_t *>(p.row_tables_dev[(size_t)s.out_tab]);
@@ -1342,8 +1398,10 @@ void plan_execute(Plan &p, const void *in, void *out) { plan_execute_sep(p, in, 
 
 void plan_execute_istft(Plan &p, const void *in, const float *window, void *out)
 {
-    for (Stage &s : p.stages)
-        if (s.kind == StageKind::Aux && s.xa.mode == AUX_ISTFT_OLA) s.xa.win = window;
+    for (Stage *s : p.launches) {
+        if (s->kind == StageKind::Istft) s->ia.win = window;
+        if (s->kind == StageKind::Aux && s->xa.mode == AUX_ISTFT_OLA) s->xa.win = window;
+    }
     plan_execute(p, in, out);
 }
 
@@ -1359,7 +1417,13 @@ void plan_execute_sep(Plan &p, const void *in, const void *in_im, void *out, voi
         Stage &s = *sp;
         void *src = resolve(p, s.in, in, out);
         void *dst = resolve(p, s.out, in, out);
-        if (s.kind == StageKind::Stockham) {
+        if (s.kind == StageKind::Istft) {
+            IstftArgs a = s.ia;
+            a.in = static_cast<const float2 *>(src);
+            a.out = static_cast<float2 *>(dst);
+            void *args[] = {&a};
+            SIP_HIP_CHECK(hipLaunchKernel(s.fused_fn, s.grid, s.block, args, s.lds, p.stream));
+        } else if (s.kind == StageKind::Stockham) {
             StockhamArgs a = s.sa;
             a.in = src;
             a.out = dst;

@@ -69,7 +69,7 @@ struct Tune {
     int rc = -1;           // rows-in / columns-out kernel for the second four-step stage
 };
 
-enum class StageKind { Stockham, Aux };
+enum class StageKind { Stockham, Aux, Istft };
 
 struct Stage {
     StageKind kind = StageKind::Stockham;
@@ -90,6 +90,8 @@ struct Stage {
     // Aux
     AuxArgs xa{};
     TableRef tab0;
+    // One-launch inverse short-time transform (fused launches only; pass twiddles in tw)
+    IstftArgs ia{};
     // Kernel of a launch that stands for several stages (Plan::fusions); null for a stage of its own
     const void *fused_fn = nullptr;
     std::string note;
@@ -190,6 +192,8 @@ const StockhamInstance *find_mfma_instance(int64_t L, int mode);
 const Stockham2dInstance *find_2d_instance(int64_t X, int64_t Y);
 // One-launch Bluestein instance of the shortest convolution of at least `min_m` points, or null.
 const BluesteinInstance *find_bluestein_instance(int64_t min_m);
+// One-launch inverse short-time transform of n-point frames, or null.
+const IstftInstance *find_istft_instance(int64_t n);
 TableRef mfma_dft_table(int mode, int sign);
 // Operand table of the single-plane K = 32 matrix passes (kernels/mfma_split.h).
 TableRef mfma2_dft_table(int mode, int sign);

@@ -62,4 +62,20 @@ const BluesteinInstance *find_bluestein_instance(int64_t min_m)
     return nullptr;
 }
 
+#define SIP_ISTFT_PART(k)                            \
+    extern const IstftInstance g_istft_part_##k[];   \
+    extern const int g_istft_part_##k##_count;
+#include "istft_parts.inc"
+#undef SIP_ISTFT_PART
+
+const IstftInstance *find_istft_instance(int64_t n)
+{
+#define SIP_ISTFT_PART(k)                                 \
+    for (int i = 0; i < g_istft_part_##k##_count; i++)    \
+        if (g_istft_part_##k[i].L == n) return &g_istft_part_##k[i];
+#include "istft_parts.inc"
+#undef SIP_ISTFT_PART
+    return nullptr;
+}
+
 }  // namespace sip

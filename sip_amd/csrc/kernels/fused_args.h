@@ -14,4 +14,25 @@ struct BluesteinInstance {
     const void *fn;
 };
 
+// One-launch inverse short-time transform (istft.h).
+struct IstftArgs {
+    const float2 *in;     // spectra (channel, n, frames)
+    float2 *out;          // samples (channel, out_len)
+    const float2 *tw;     // pass twiddles of the inverse n-point FFT
+    const float *win;     // window, n values
+    int64_t frames, hop, out_len;
+    int64_t start;        // first sample of the overlap-add span that is written
+    int64_t tiles;        // tiles per channel
+    int64_t keep;         // frames a tile advances by
+    int32_t halo;         // frames of a tile that the tile before ends: ceil(n / hop) - 1
+    int32_t F, LP;        // frames per tile, LDS pitch of a frame
+    FastDiv div_F, div_tiles, div_hop;
+};
+
+struct IstftInstance {
+    int32_t L, T, npass;
+    int32_t radix[8];
+    const void *fn;
+};
+
 }  // namespace sip

@@ -291,10 +291,42 @@ REAL_ROWS_LONG = {8640, 9000, 9216, 9375, 9600, 9720, 10000, 10125, 10240, 10368
 RC_MIN_THREADS = 8
 
 
+# One-launch inverse short-time transforms (istft.h): every 2,3,5-smooth frame length in this range,
+# with the leaf's radix sequence and threads.
+ISTFT_MIN, ISTFT_MAX, ISTFT_PARTS = 24, 1499, 6
+
+
+def istft_instances():
+    return [(n, t, seq) for n, t, seq in instances()
+            if ISTFT_MIN <= n <= ISTFT_MAX and all(r not in (7, 11, 13) for r in seq)]
+
+
+def write_if_changed(path, text):
+    if not os.path.exists(path) or open(path).read() != text:
+        with open(path, "w") as fh:
+            fh.write(text)
+
+
+def write_istft(outdir):
+    inst = istft_instances()
+    for k in range(ISTFT_PARTS):
+        lines = ["// Generated by gen_instances.py: one-launch inverse short-time transforms (do not edit).",
+                 '#include "istft.h"', "namespace sip {", f"extern const IstftInstance g_istft_part_{k}[] = {{"]
+        items = inst[k::ISTFT_PARTS]
+        for n, t, seq in items:
+            rs = ", ".join(str(r) for r in seq)
+            lines.append(f"    {{{n}, {t}, {len(seq)}, {{{rs}}}, (const void *)&istft_kernel<{n}, {t}, {rs}>}},")
+        lines += ["};", f"extern const int g_istft_part_{k}_count = {len(items)};", "}  // namespace sip"]
+        write_if_changed(os.path.join(outdir, f"istft_part_{k}.hip"), "\n".join(lines) + "\n")
+    inc = ["// Generated by gen_instances.py (do not edit)."] + [f"SIP_ISTFT_PART({k})" for k in range(ISTFT_PARTS)]
+    write_if_changed(os.path.join(outdir, "istft_parts.inc"), "\n".join(inc) + "\n")
+
+
 def main():
     outdir = sys.argv[1]
     nparts = int(sys.argv[2])
     os.makedirs(outdir, exist_ok=True)
+    write_istft(outdir)
     inst = instances()
     parts = [[] for _ in range(nparts)]
     # balance by estimated code size (passes x length)
@@ -364,19 +396,11 @@ def main():
         lines.append("};")
         lines.append(f"extern const int g_stockham_part_{k}_count = {len(items)};")
         lines.append("}  // namespace sip")
-        path = os.path.join(outdir, f"stockham_part_{k}.hip")
-        text = "\n".join(lines) + "\n"
-        if not os.path.exists(path) or open(path).read() != text:
-            with open(path, "w") as fh:
-                fh.write(text)
+        write_if_changed(os.path.join(outdir, f"stockham_part_{k}.hip"), "\n".join(lines) + "\n")
     inc = ["// Generated by gen_instances.py (do not edit)."]
     for k in range(nparts):
         inc.append(f"SIP_STOCKHAM_PART({k})")
-    text = "\n".join(inc) + "\n"
-    path = os.path.join(outdir, "stockham_parts.inc")
-    if not os.path.exists(path) or open(path).read() != text:
-        with open(path, "w") as fh:
-            fh.write(text)
+    write_if_changed(os.path.join(outdir, "stockham_parts.inc"), "\n".join(inc) + "\n")
     print(f"{len(inst)} leaf lengths in {nparts} parts")
 
 

@@ -1,4 +1,4 @@
-"""Launches that stand for several stages of a plan (one-launch Bluestein): each
+"""Launches that stand for several stages of a plan (one-launch Bluestein, one-launch ISTFT): each
 against the FP64 oracle (rel-L2 5e-6 for Bluestein lengths, 2e-6 otherwise) and against the stages run
 one by one (SIP_FFT_FUSE=0 at plan time). Both ways round a result a few times per pass of log2 M
 levels, each within 4e-7 of the exact one, so they agree to 1e-6.
@@ -104,3 +104,25 @@ def test_bluestein_split_planes(torch_cuda, monkeypatch, n, b):
 
     got, staged = _both(lambda h: h.make_plan_1d(n, S.ASCEND_FFT_C2C_SEP, INV, b), execute, monkeypatch)
     _agree(f"bluestein split {n} x {b}", got, staged, oracle.c2c(x, sign_of(INV)), 5e-6)
+
+
+# one frame more than a tile holds, fewer frames than the halo, hops that divide the frame and that do
+# not, no overlap at all, odd lengths, the shortest hop that is still one launch (n / 8 with 16 frames)
+@pytest.mark.parametrize("ch,n,hop,frames", [(1, 24, 6, 65), (2, 27, 10, 40), (3, 256, 64, 2), (2, 256, 256, 70),
+                                             (2, 400, 160, 131), (1, 625, 125, 9), (2, 1024, 256, 17),
+                                             (1, 1024, 128, 33), (2, 1080, 270, 20), (1, 1458, 365, 12)])
+def test_istft_one_launch(torch_cuda, monkeypatch, ch, n, hop, frames):
+    import torch
+    rng = np.random.default_rng(n * 7 + hop)
+    x = (rng.standard_normal((ch, n, frames)) + 1j * rng.standard_normal((ch, n, frames))).astype(np.complex64)
+    w = (np.hanning(n + 2)[1:-1] + 0.05).astype(np.float32)
+    xd, wd = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()
+    y = torch.empty((ch, oracle.istft_out_len(n, hop, frames)), dtype=torch.complex64, device="cuda")
+
+    def execute(h):
+        assert h.exec_istft(xd, wd, y) == S.ACL_SUCCESS
+        torch.cuda.synchronize()
+        return y.cpu().numpy()
+
+    got, staged = _both(lambda h: h.istft_make_plan(xd, n, hop, n), execute, monkeypatch)
+    _agree(f"istft ch={ch} n={n} hop={hop} frames={frames}", got, staged, oracle.istft(x, n, hop, w), 2e-6)
