@@ -381,6 +381,15 @@ static int lds_pitch(int64_t n)
     return lp | 1;
 }
 
+// Column tiles of this length on one LDS plane: SIP_FFT_SPLIT_COLS=0 never, 1 power-of-two lengths, 2
+// (default) every length.
+static bool split_columns(int64_t L)
+{
+    const char *e = std::getenv("SIP_FFT_SPLIT_COLS");
+    const int mode = e ? std::atoi(e) : 2;
+    return mode == 2 || (mode == 1 && (L & (L - 1)) == 0);
+}
+
 constexpr int64_t kFillWorkgroups = 512;  // two workgroups per CU of MI355X (256 CUs)
 
 struct Builder {
@@ -428,6 +437,21 @@ struct Builder {
                env_flag("SIP_FFT_BIG_LEAF", true);
     }
 
+    // Columns of 1025 to 4096 points in one pass of the long column kernels instead of the two four-step
+    // passes, from 128 tiles up (half of the CUs). Measured on MI355X, two passes / one, 64 MiB of columns:
+    // 1080 60 / 35 us, 2048 56 / 30, 4096 54 / 42; fewer tiles leave the chip to a few long workgroups: 2048
+    // x 100 columns (7 tiles) 9 / 19 us, R2C 1080 x 1920 (61 tiles) 26 / 28 us, C2C 2048 x 2048 (128) 44 / 37.
+    bool long_columns(int64_t L, const Lay &in, const Lay &out) const
+    {
+        const ColumnInstance *ci = L > kColumnLeafMax ? find_column_instance(L, false) : nullptr;
+        bool ok = true;
+        int tab;
+        return ci && p.precision == PREC_FP32 && !is_user(in.buf) && !is_user(out.buf) &&
+               to_tile(in, &ok, &tab).unit_f && to_tile(out, &ok, &tab).unit_f && ok &&
+               count(normalize(in.dims)) >= 128 * (int64_t)ci->F && split_columns(L) &&
+               env_flag("SIP_FFT_COL_DIRECT", true);
+    }
+
     void add_stockham(int64_t L, int sign, const Lay &in, const Lay &out, int io_mode, int64_t in_len,
                       int64_t out_len, int64_t tw4_ntot, int64_t col_div, const std::string &note)
     {
@@ -439,9 +463,17 @@ struct Builder {
         const StockhamInstance *mf = (p.precision != PREC_FP32 && io_mode == IO_C2C && !in_sep && !out_sep)
                                          ? find_mfma_instance(L, p.precision) : nullptr;
         if (mf) inst = mf;
-        if (!inst) throw SipError(AsdSip::ACL_ERROR_API_NOT_SUPPORT, "no kernel for length " + std::to_string(L));
         bool ok = true;
         Stage st;
+        const TileDesc tin = to_tile(in, &ok, &st.in_tab), tout = to_tile(out, &ok, &st.out_tab);
+        // column tiles (C2C, strided on both sides): first / last pass straight from / to HBM with
+        // lanes walking adjacent columns, on the column kernels' own threads and radices. The tuning
+        // switches that stage them through LDS or on two planes keep the leaf.
+        const bool columns = io_mode == IO_C2C && tin.unit_f && tout.unit_f && !in_sep && !out_sep &&
+                             env_flag("SIP_FFT_COL_DIRECT", true);
+        const ColumnInstance *ci = columns && !mf && split_columns(L) ? find_column_instance(L, tw4_ntot != 0) : nullptr;
+        if (ci) inst = &ci->inst;
+        if (!inst) throw SipError(AsdSip::ACL_ERROR_API_NOT_SUPPORT, "no kernel for length " + std::to_string(L));
         st.kind = StageKind::Stockham;
         st.in = in.buf;
         st.out = out.buf;
@@ -449,8 +481,8 @@ struct Builder {
         st.sign = sign;
         StockhamArgs &a = st.sa;
         std::memset(&a, 0, sizeof(a));
-        a.tin = to_tile(in, &ok, &st.in_tab);
-        a.tout = to_tile(out, &ok, &st.out_tab);
+        a.tin = tin;
+        a.tout = tout;
         if (!ok) throw SipError(AsdSip::ACL_ERROR_API_NOT_SUPPORT, "layout has more than 3 batch dimensions");
         const int64_t nfft = count(normalize(in.dims));
         if (nfft != count(normalize(out.dims)))
@@ -467,7 +499,7 @@ struct Builder {
         a.LP = lp;
         const int T = inst->T;
         const bool column = a.tin.unit_f || a.tout.unit_f;
-        const size_t per = (size_t)2 * lp * 4 + 24;
+        const size_t per = ci ? (size_t)lp * 4 : (size_t)2 * lp * 4 + 24;
         int F;
         if (column) {
             // Tile width: a multiple of 16 transforms (each row run covers whole 128-byte lines),
@@ -482,8 +514,11 @@ struct Builder {
             // C2C rows: 43200 x 1056 459 -> 401 us, 36000 x 864 350 -> 277 us, 27000 x 604
             // 168 -> 154 us; power-of-two columns keep the wider tiles (the 256-row stage B of
             // 64000 x 635: 360 us at 32 wide, 393 us at 16).
+            // A tile of one wave or less takes a whole one (20 x 419430, one thread per column: 34 us at
+            // 16 wide, 22 us at 64).
             const bool pow2 = (L & (L - 1)) == 0;
-            F = want > 0 ? want : (pow2 ? std::min(64, std::max(16, (512 / T) & ~15)) : 16);
+            if (want <= 0 && ci) want = ci->F;
+            F = want > 0 ? want : pow2 ? std::min(64, std::max(16, (512 / T) & ~15)) : T >= 4 ? 16 : T >= 2 ? 32 : 64;
             if (F >= 16) F &= ~15;
             while (F > 1 && ((size_t)F * per > 160 * 1024 || F * T > 1024)) F /= 2;
         } else {
@@ -547,10 +582,7 @@ struct Builder {
             a.tout.vec2 = 0;
         }
         const bool rows = io_mode == IO_C2C && a.direct_in && a.direct_out && inst->rows_fwd != nullptr;
-        // column tiles (C2C, strided on both sides): first / last pass straight from / to HBM with
-        // lanes walking adjacent columns
-        a.col_direct = (io_mode == IO_C2C && a.tin.unit_f && a.tout.unit_f && (!mf || mf_cols) && !in_sep && !out_sep &&
-                        env_flag("SIP_FFT_COL_DIRECT", true)) ? 1 : 0;
+        a.col_direct = columns && (!mf || mf_cols) ? 1 : 0;
         // Single-plane exchange (half the LDS, twice the resident workgroups) by default for rows
         // with 32 or more threads per transform. Measured on MI355X, 1 GiB of C2C rows: 4096
         // 373 us against 397 us, 1024 370 / 395, 8192 428 / 497, 16384 436 / 646; at 16 threads
@@ -571,12 +603,7 @@ struct Builder {
         // with 16-wide mixed-length tiles and the derived four-step twiddles, mixed lengths gain
         // too: four-step 43200 x 1056 387-399 -> 346 us, 64000 x 635 370 -> 337 us, 2D 1000^2 x 64
         // 528-535 -> 500 us, 3D 240^3 x 8 1155 -> 1086 us.
-        {
-            const char *e = std::getenv("SIP_FFT_SPLIT_COLS");
-            const int mode = e ? std::atoi(e) : 2;  // 0 never, 1 power-of-two lengths, 2 every length
-            if (a.col_direct && inst->cols[0] != nullptr && (mode == 2 || (mode == 1 && (L & (L - 1)) == 0)))
-                a.split_lds = 1;
-        }
+        if (a.col_direct && (ci || (mf && split_columns(L)))) a.split_lds = 1;
         // Fused real transforms on contiguous rows: single plane as well (pair pre-process read
         // straight from HBM for C2R, post-process through the plane for R2C). Measured on MI355X:
         // 8192 x 4096 R2C 58.1 -> 47.5 us, C2R 58.8 -> 46.7 us; 12000 x 2048 77 / 82 -> 68 / 67 us;
@@ -595,7 +622,14 @@ struct Builder {
             a.split_lds = 0;
             a.col_direct = 0;
         }
-        a.xcd_remap = p.tune.xcd >= 0 ? p.tune.xcd == 1 : env_flag("SIP_FFT_XCD", false);
+        // Workgroups go round robin to the 8 XCDs, each with its own L2. Where a column tile's runs do not
+        // start on 128-byte lines (a stride that is not a multiple of 16 elements), adjacent tiles share
+        // lines, which two L2s would fetch and write apart: XCD-contiguous tile order. Measured on
+        // MI355X, launch / XCD-contiguous order, columns of 64 MiB: 100 x 83886 35.2 / 26.7 us, 243 x
+        // 34521 38.9 / 28.1, 1080 x 7767 42.4 / 36.8, R2C 512^2 x 64 68.9 / 54.9; whole lines lose by it:
+        // 256 x 32768 22.8 / 25.0, 1024 x 8192 25.8 / 27.9.
+        const bool split_lines = (a.tin.unit_f && a.tin.es % 16 != 0) || (a.tout.unit_f && a.tout.es % 16 != 0);
+        a.xcd_remap = p.tune.xcd >= 0 ? p.tune.xcd == 1 : env_flag("SIP_FFT_XCD", column && split_lines);
         // matrix passes read [k][16] twiddle rows; the single-plane rows kernel (K = 32) reads the
         // interleaved operand table, the two-plane tile (K = 16) the blocked one
         const bool mf2 = mf != nullptr && a.split_lds;
@@ -784,6 +818,7 @@ struct Builder {
                 }
         }
         if (!L1) throw SipError(AsdSip::ACL_ERROR_API_NOT_SUPPORT, "cannot split length " + std::to_string(L));
+        const size_t first = p.stages.size();
         // mid layout: same structure as the input; in place when the input may be overwritten and
         // the final store does not go back into that same buffer (stage B is not in-place safe)
         Lay mid = in;
@@ -813,6 +848,13 @@ struct Builder {
         Lay bin{mid.buf, mid.es, with_dim(mid.dims, posB, {L1, mid.es * L2})};
         Lay bout{out.buf, out.es * L1, with_dim(out.dims, posB, {L1, out.es})};
         axis(L2, sign, bin, bout, true, depth + 1);
+        if (depth == 0 && forced <= 1 && fusing() && long_columns(L, in, out)) {
+            const size_t last = p.stages.size() - 1;
+            add_stockham(L, sign, in, out, IO_C2C, L, L, 0, 1, "columns " + std::to_string(L));
+            Stage st = std::move(p.stages.back());
+            p.stages.pop_back();
+            p.fusions.push_back(Fusion{first, last, std::move(st)});
+        }
     }
 
     void bluestein(int64_t N, int sign, const Lay &in, const Lay &out)
@@ -1273,17 +1315,33 @@ void plan_materialize_external(Plan &p, const std::vector<const int64_t *> &dev_
 // 2D 1024^2 x 128 855 -> 837 us, 3D 128^3 x 64 801 -> 786 us, 32768 x 4096 540 -> 532 us, but
 // slower on inputs that the last-level cache still holds (2000 x 8192 45 -> 56 us, R2C 8192 x 4096
 // 48 -> 52 us, four-step 43200 x 1056 341 -> 359 us, batching workload 8.9 -> 9.3 ms), hence the
-// size threshold.
+// size threshold. A plan of several launches loads its input nontemporally already when what one
+// execution touches (input, intermediates, output) is more than half of that cache: the input is most
+// likely not in it (a program's other data between two calls is as large), and loading it past the cache
+// keeps the intermediate there for the next launch. On three buffer sets in turn / on one set over and
+// over, cached -> nontemporal: 1048576 x 8 72.6 -> 54.2 / 53.3 -> 54.9 us, 65536 x 128 54.7 -> 50.3 / 47.9 ->
+// 52.0, 1000000 x 8 85.0 -> 78.4 / 77.5 -> 78.0, 100000 x 83 74.2 -> 70.0 / 65.7 -> 69.9.
 void plan_mark_streaming(Plan &p)
 {
     const bool on_out = env_flag("SIP_FFT_NT_OUT", true), on_in = env_flag("SIP_FFT_NT_IN", true);
     constexpr int64_t kNtInBytes = int64_t(512) << 20;
-    for (size_t i = 0; i < p.stages.size(); i++) {
-        Stage &s = p.stages[i];
+    constexpr int64_t kNtInFootprint = int64_t(128) << 20;
+    const std::vector<Stage *> run = plan_launches(p);
+    const bool gathered = !p.row_tables.empty() || !p.external_tables.empty();
+    int64_t footprint = 0;  // bytes read by the first launch and written outside in-place steps
+    for (size_t i = 0; i < run.size(); i++) {
+        const StockhamArgs &a = run[i]->sa;
+        if (run[i]->kind != StageKind::Stockham) continue;
+        if (i == 0) footprint += a.nfft * (int64_t)a.in_len * 8;
+        if (run[i]->in.kind != run[i]->out.kind || run[i]->in.ws_index != run[i]->out.ws_index)
+            footprint += a.nfft * (int64_t)a.out_len * 8;
+    }
+    for (size_t i = 0; i < run.size(); i++) {
+        Stage &s = *run[i];
         if (s.kind != StageKind::Stockham) continue;
         bool read_later = false;
-        for (size_t j = i + 1; j < p.stages.size(); j++) {
-            const BufRef &in = p.stages[j].in;
+        for (size_t j = i + 1; j < run.size(); j++) {
+            const BufRef &in = run[j]->in;
             if (in.kind == s.out.kind && (in.kind == BUF_IN || in.kind == BUF_OUT || in.ws_index == s.out.ws_index))
                 read_later = true;
         }
@@ -1301,14 +1359,15 @@ void plan_mark_streaming(Plan &p)
         // 512^2 x 256 394 -> 352 us, 3D 128^3 x 64 778 -> 758 us, but the batching form's graph
         // 8.9 -> 9.5 ms with them on its groups' final stores
         const bool cols_out = s.sa.tout.unit_f != 0;
-        const bool gathered = !p.row_tables.empty() || !p.external_tables.empty();
         const int64_t out_bytes = s.sa.nfft * (int64_t)s.sa.out_len * 8;
         const bool aligned_out = cols_out ? (s.sa.F % 16 == 0 && s.sa.tout.es % 16 == 0 && s.sa.tw4_ntot == 0 &&
                                              !gathered && out_bytes >= kNtInBytes)
                                           : rows_aligned_out;
         s.sa.nt_out = (on_out && !read_later && aligned_out) ? 1 : 0;
         const int64_t in_bytes = s.sa.nfft * (int64_t)s.sa.in_len * 8;
-        s.sa.nt_in = (on_in && s.sa.io_mode == IO_C2C && in_bytes >= kNtInBytes && aligned_in) ? 1 : 0;
+        const bool cold = i == 0 && run.size() > 1 && s.in.kind == BUF_IN && !gathered && footprint > kNtInFootprint &&
+                          (!cols_in || s.sa.tin.es % 8 == 0);
+        s.sa.nt_in = (on_in && s.sa.io_mode == IO_C2C && (in_bytes >= kNtInBytes || cold) && aligned_in) ? 1 : 0;
     }
 }
 

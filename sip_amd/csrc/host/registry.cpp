@@ -62,6 +62,27 @@ const BluesteinInstance *find_bluestein_instance(int64_t min_m)
     return nullptr;
 }
 
+#define SIP_COLUMNS_PART(k)                              \
+    extern const ColumnInstance g_columns_part_##k[];    \
+    extern const int g_columns_part_##k##_count;
+#include "columns_parts.inc"
+#undef SIP_COLUMNS_PART
+
+const ColumnInstance *find_column_instance(int64_t L, bool tw4)
+{
+    static const auto m = [] {
+        std::map<std::pair<int64_t, bool>, const ColumnInstance *> r;
+#define SIP_COLUMNS_PART(k)                                         \
+    for (int i = 0; i < g_columns_part_##k##_count; i++)            \
+        r[{g_columns_part_##k[i].inst.L, g_columns_part_##k[i].inst.cols[2] != nullptr}] = &g_columns_part_##k[i];
+#include "columns_parts.inc"
+#undef SIP_COLUMNS_PART
+        return r;
+    }();
+    auto it = m.find({L, tw4});
+    return it == m.end() ? nullptr : it->second;
+}
+
 #define SIP_ISTFT_PART(k)                            \
     extern const IstftInstance g_istft_part_##k[];   \
     extern const int g_istft_part_##k##_count;

@@ -14,6 +14,9 @@ from __future__ import annotations
 import os
 import sys
 
+sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))  # also when loaded from a path
+from column_shapes import COLUMN_SHAPES, COLUMN_TW_SHAPES, LONG_COLUMN_SHAPES
+
 MAX_SMOOTH = 16384
 MAX_POW2 = 16384
 MAX_PRIME_FACTOR_LEN = 4096
@@ -274,9 +277,46 @@ def instances():
 # 15552 169 / 158; every other length from 4320 to 16384 is faster on one plane (up to 1.7x).
 ROWS_TWO_PLANE = {8748, 12000, 12150, 12960, 14580, 15000, 15552, 15625, 16200}
 
-# longest leaf used for column tiles (the host's kColumnLeafMax): these lengths also get the
-# single-plane column-tile kernel
+# longest leaf used for column tiles (the host's kColumnLeafMax); every leaf up to it gets a column
+# kernel of its own (columns.h) with the shape measured for that role (column_shapes.py)
 COLUMN_LEAF_MAX = 1024
+COLUMN_PARTS = 16
+def column_instances():
+    """(length, four-step twiddle, threads, radices, waves per SIMD or 0, columns per tile or 0 for the
+    planner's rule)."""
+    out = []
+    for n, t, seq in instances():
+        if n <= COLUMN_LEAF_MAX:
+            for tw, shapes in ((False, COLUMN_SHAPES), (True, COLUMN_TW_SHAPES)):
+                out.append((n, tw) + tuple(shapes.get(n, (t, seq, 0))) + (0,))
+    out += [(n, False) + shape for n, shape in LONG_COLUMN_SHAPES.items()]
+    for n, _, t, seq, _, f in out:
+        p = 1
+        for r in seq:
+            p *= r
+        assert p == n and elems_per_thread(n, seq, t) <= 40 and (f or 1) * t <= 1024, (n, t, seq)
+    return sorted(out)
+
+
+def write_columns(outdir):
+    inst = column_instances()
+    for k in range(COLUMN_PARTS):
+        items = inst[k::COLUMN_PARTS]
+        lines = ["// Generated by gen_instances.py: column-tile kernels (do not edit).", '#include "columns.h"',
+                 "namespace sip {", f"extern const ColumnInstance g_columns_part_{k}[] = {{"]
+        for n, tw, t, seq, w, f in items:
+            rs = ", ".join(str(r) for r in seq)
+            names = [f"(const void *)&stockham_cols_kernel<{w}, {n}, {t}, {sg}, {str(tw).lower()}, {rs}>"
+                     for sg in (-1, 1)]
+            cols = ", ".join(["nullptr, nullptr"] * tw + names + ["nullptr, nullptr"] * (not tw))
+            lines.append(f"    {{{{{n}, {t}, {len(seq)}, {{{rs}}}, nullptr, nullptr, nullptr, nullptr, "
+                         f"{{{cols}}}, {{nullptr, nullptr, nullptr, nullptr}}, {{nullptr, nullptr}}}}, {f}}},")
+        lines += ["};", f"extern const int g_columns_part_{k}_count = {len(items)};", "}  // namespace sip"]
+        write_if_changed(os.path.join(outdir, f"columns_part_{k}.hip"), "\n".join(lines) + "\n")
+    inc = ["// Generated by gen_instances.py (do not edit)."] + [f"SIP_COLUMNS_PART({k})" for k in range(COLUMN_PARTS)]
+    write_if_changed(os.path.join(outdir, "columns_parts.inc"), "\n".join(inc) + "\n")
+
+
 # half lengths (with 32 or more threads per transform) of the real transforms that also get
 # single-plane R2C / C2R row kernels: every one up to 8192, and those above 8192 where the single
 # plane measured faster than the two-plane fused kernel on MI355X (R2C + C2R of 256 MiB of reals,
@@ -327,6 +367,7 @@ def main():
     nparts = int(sys.argv[2])
     os.makedirs(outdir, exist_ok=True)
     write_istft(outdir)
+    write_columns(outdir)
     inst = instances()
     parts = [[] for _ in range(nparts)]
     # balance by estimated code size (passes x length)
@@ -367,14 +408,6 @@ def main():
                 rows = f"(const void *)&{rf}, (const void *)&{ri}"
             else:
                 rows = "nullptr, nullptr"
-            if n <= COLUMN_LEAF_MAX:
-                names = [f"stockham_cols_kernel<{n}, {t}, {sg}, {tw4}, {rs}>" for tw4 in ("false", "true")
-                         for sg in (-1, 1)]
-                for nm in names:
-                    lines.append(f"template __global__ void {nm}(const StockhamArgs);")
-                cols = "{" + ", ".join(f"(const void *)&{nm}" for nm in names) + "}"
-            else:
-                cols = "{nullptr, nullptr, nullptr, nullptr}"
             if t >= 32 and (n <= REAL_ROWS_MAX or n in REAL_ROWS_LONG):
                 names = [f"stockham_real_rows_kernel<{n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)]
                 for nm in names:
@@ -389,7 +422,8 @@ def main():
                 rc = "{" + ", ".join(f"(const void *)&{nm}" for nm in names) + "}"
             else:
                 rc = "{nullptr, nullptr}"
-            tab.append(f"    {{{n}, {t}, {len(seq)}, {{{radix}}}, (const void *)&{kf}, (const void *)&{ki}, {rows}, {cols}, "
+            tab.append(f"    {{{n}, {t}, {len(seq)}, {{{radix}}}, (const void *)&{kf}, (const void *)&{ki}, {rows}, "
+                       "{nullptr, nullptr, nullptr, nullptr}, "
                        f"{real}, {rc}}},")
         lines.append(f"extern const StockhamInstance g_stockham_part_{k}[] = {{")
         lines += tab

@@ -107,11 +107,19 @@ struct StockhamInstance {
     const void *rows_fwd;    // single-plane contiguous-row kernels (T >= 16 only, else null)
     const void *rows_inv;
     const void *cols[4];     // single-plane column-tile kernels, fwd / inv without and fwd / inv
-                             // with the four-step twiddle (L <= 1024 only, else null)
+                             // with the four-step twiddle (column and matrix-core instances only)
     const void *real_rows[4];  // single-plane R2C fwd / inv, C2R fwd / inv rows (T >= 32; L <= 8192
                                // and the longer L where they measured faster; else null)
     const void *rc[2];         // single-plane rows-in / columns-out fwd / inv (four-step second
                                // stage; L <= 1024 with two or more passes and T >= 8, else null)
+};
+
+// Column-tile kernels of one length, with the threads and radices measured for that role: `inst` holds
+// L, T, the radices and cols[] only. The kernels with the four-step twiddle on store have an entry of
+// their own (cols[2..3]; lengths up to 1024), those without another (cols[0..1]; up to 4096).
+struct ColumnInstance {
+    StockhamInstance inst;
+    int32_t F;  // columns per tile; 0 = the planner's rule
 };
 
 // Registry entry of a fused 2D tile instance (stockham2d.h). The radix sequences, and so the

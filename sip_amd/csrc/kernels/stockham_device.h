@@ -730,15 +730,6 @@ __device__ __forceinline__ void split_cols(const StockhamArgs &a, float *pl, int
     split_chain<L, T, S, 1, R0, Rest...>(pl, a.tw, flp * a.LP, t, active, v, io);
 }
 
-// Column tiles, single LDS plane (separate kernel so that its register budget is its own); TW4:
-// the stage applies the four-step twiddle on store.
-template <int L, int T, int S, bool TW4, int... Rs>
-__global__ __launch_bounds__(1024) void stockham_cols_kernel(const StockhamArgs a)
-{
-    extern __shared__ float lds[];
-    split_cols<L, T, S, TW4, Rs...>(a, lds, tile_index(a));
-}
-
 // Rows in, columns out (the second stage of a four-step split: transform k1 is a contiguous row of
 // the intermediate and its element k2 goes to k1 + L1 k2, so adjacent transforms are adjacent on
 // output). The first pass reads each row straight from HBM with the transform's T threads on

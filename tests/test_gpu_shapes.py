@@ -1,0 +1,76 @@
+"""Kernels whose threads and radices were chosen per role and length (column_shapes.py): every listed length
+against the FP64 oracle (rel-L2 2e-6), on counts that leave the last tile partly empty and, for columns,
+strides that do not fall on whole 128-byte lines."""
+import importlib.util
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+import sip_amd as S
+from fftcase import FWD, INV, c2c, make, report, sign_of
+
+pytestmark = pytest.mark.gpu
+TOL = 2e-6
+
+
+def _shapes(module):
+    path = os.path.join(S.HERE, "csrc", "kernels", module + ".py")
+    spec = importlib.util.spec_from_file_location(module, path)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+    return mod
+
+
+COLS = _shapes("column_shapes")
+
+
+def _vertical(n, b, direction):
+    x = oracle.uniform_complex((n, b), 0x5EED0E00 + n)
+    y = c2c(x.reshape(n, b), [n], direction, S.ASCEND_FFT_VERTICAL)
+    want = oracle.c2c(np.ascontiguousarray(x.T), sign_of(direction)).T
+    rel, _ = report(f"columns {n} x {b}", y, want)
+    assert rel <= TOL
+
+
+@pytest.mark.parametrize("n", sorted(COLS.COLUMN_SHAPES) + [20, 24, 45])
+def test_column_shapes(torch_cuda, n):
+    _vertical(n, 37, INV if n % 3 else FWD)
+
+
+@pytest.mark.parametrize("n", sorted(COLS.LONG_COLUMN_SHAPES))
+def test_long_column_shapes(torch_cuda, n):
+    """One pass from 128 tiles up (an odd count: 2051 columns), two below; both checked."""
+    h = make([n], S.ASCEND_FFT_C2C, FWD, 2051, S.ASCEND_FFT_VERTICAL)
+    assert h.describe()["fused"][0]["note"] == f"columns {n}"
+    h.destroy()
+    _vertical(n, 2051, FWD if n % 2 else INV)
+    _vertical(n, 19, INV)
+
+
+@pytest.mark.parametrize("n", sorted(COLS.COLUMN_TW_SHAPES))
+def test_column_shapes_with_twiddle(torch_cuda, monkeypatch, n):
+    """First four-step stage of length n (forced factor), second stage the shortest smooth leaf that makes the
+    length one that no single launch takes."""
+    m = next(v for v in S.smooth_lengths(33, 1024) if v * n > 32768)
+    monkeypatch.setenv("SIP_FFT_SPLIT_L1", str(n))
+    d = INV if n % 3 else FWD
+    x = oracle.uniform_complex((3, n * m), 0x5EED0F00 + n)
+    h = make([n * m], S.ASCEND_FFT_C2C, d, 3)
+    st = h.describe()["stages"][0]
+    assert st["L"] == n and st["tw4"] == n * m and st["T"] == COLS.COLUMN_TW_SHAPES[n][0]
+    h.destroy()
+    y = c2c(x, [n * m], d)
+    rel, _ = report(f"four-step {n} x {m}", y, oracle.c2c(x, sign_of(d)))
+    assert rel <= TOL
+
+
+def test_streaming_input_of_several_launches(torch_cuda):
+    """A plan of several launches that touches more than 128 MiB loads its input nontemporally."""
+    h = make([1 << 20], S.ASCEND_FFT_C2C, FWD, 8)
+    assert [s["nt_in"] for s in h.describe()["stages"]] == [1, 0]
+    h.destroy()
+    h = make([1 << 20], S.ASCEND_FFT_C2C, FWD, 5)
+    assert [s["nt_in"] for s in h.describe()["stages"]] == [0, 0]
+    h.destroy()
