@@ -243,7 +243,7 @@ std::vector<Tune> candidates(int64_t n)
     if (inst && n <= 16384) {
         for (int sl : {0, 1})
             for (int x : {0, 1}) {
-                if (sl == 1 && !inst->rows_fwd) continue;
+                if (sl == 1 && !find_role(ROLE_ROWS, n)) continue;
                 Tune t;
                 t.split_lds = sl;
                 t.xcd = x;

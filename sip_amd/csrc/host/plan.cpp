@@ -421,10 +421,8 @@ struct Builder {
 
     bool leaf_ok(int64_t L, const Lay &in, const Lay &out) const
     {
-        const StockhamInstance *inst = find_instance(L);
-        if (!inst) return false;
-        if (is_column(in) || is_column(out)) return L <= kColumnLeafMax;
-        if (L <= kRowLeafMax) return true;
+        if (is_column(in) || is_column(out)) return L <= kColumnLeafMax && find_instance(L);
+        if (L <= kRowLeafMax) return find_instance(L) != nullptr;
         // Lengths above 16384 (2,3,5-smooth, up to 32768): one workgroup of up to 1024 threads per
         // transform on the single-plane rows kernel (plane of 4 (L + L/16 + 1) bytes <= 136 KiB),
         // for contiguous interleaved FP32 rows on both sides, from 256 transforms up (one
@@ -432,7 +430,7 @@ struct Builder {
         // against the two four-step launches: 32768 x 4096 0.54 / 0.81 ms, 20000 x 6710 0.83 /
         // 1.39 ms, 30375 x 4418 1.11 / 1.55 ms; with few transforms the split's parallelism wins
         // (32768 x 16 23 / 14 us, 20000 x 64 25 / 20 us).
-        return inst->rows_fwd != nullptr && in.es == 1 && out.es == 1 && !is_user(in.buf) && !is_user(out.buf) &&
+        return find_role(ROLE_ROWS, L) && in.es == 1 && out.es == 1 && !is_user(in.buf) && !is_user(out.buf) &&
                p.precision == PREC_FP32 && p.big_leaf && count(normalize(in.dims)) >= big_leaf_min_rows(p) &&
                env_flag("SIP_FFT_BIG_LEAF", true);
     }
@@ -443,7 +441,7 @@ struct Builder {
     // x 100 columns (7 tiles) 9 / 19 us, R2C 1080 x 1920 (61 tiles) 26 / 28 us, C2C 2048 x 2048 (128) 44 / 37.
     bool long_columns(int64_t L, const Lay &in, const Lay &out) const
     {
-        const ColumnInstance *ci = L > kColumnLeafMax ? find_column_instance(L, false) : nullptr;
+        const RoleInstance *ci = L > kColumnLeafMax ? find_role(ROLE_COLS, L) : nullptr;
         bool ok = true;
         int tab;
         return ci && p.precision == PREC_FP32 && !is_user(in.buf) && !is_user(out.buf) &&
@@ -471,8 +469,26 @@ struct Builder {
         // switches that stage them through LDS or on two planes keep the leaf.
         const bool columns = io_mode == IO_C2C && tin.unit_f && tout.unit_f && !in_sep && !out_sep &&
                              env_flag("SIP_FFT_COL_DIRECT", true);
-        const ColumnInstance *ci = columns && !mf && split_columns(L) ? find_column_instance(L, tw4_ntot != 0) : nullptr;
-        if (ci) inst = &ci->inst;
+        // Contiguous rows of plain C2C stages: the row kernels' own threads and radices (every first and last
+        // pass straight from / to HBM), unless the tuner or SIP_FFT_SPLIT_LDS=0 asks for the two-plane leaf.
+        const bool flat_in = tin.es == 1 && !tin.unit_f && !in_sep, flat_out = tout.es == 1 && !tout.unit_f && !out_sep;
+        const RoleInstance *role = nullptr;
+        if (columns && !mf && split_columns(L))
+            role = find_role(tw4_ntot != 0 ? ROLE_COLS_TW : ROLE_COLS, L);
+        else if (io_mode == IO_C2C && !mf && flat_in && flat_out && tw4_ntot == 0 && (L > kRowLeafMax || p.tune.split_lds != 0) &&
+                 (L > kRowLeafMax || env_flag("SIP_FFT_SPLIT_LDS", true)))
+            role = find_role(ROLE_ROWS, L);
+        else if ((io_mode == IO_R2C_EVEN || io_mode == IO_C2R_EVEN) && flat_in && flat_out && env_flag("SIP_FFT_SPLIT_REAL", true))
+            role = find_role(ROLE_REAL_ROWS, L);
+        // Rows in, columns out (the second four-step stage: contiguous rows of the intermediate,
+        // transposed store): one plane, the first pass straight from HBM along each row, the last
+        // pass straight to HBM across adjacent transforms (instead of the two-plane tile with
+        // LDS-staged store).
+        else if (io_mode == IO_C2C && !mf && flat_in && tout.unit_f && !out_sep && tw4_ntot == 0 &&
+                 (p.tune.rc >= 0 ? p.tune.rc == 1 : env_flag("SIP_FFT_RC", true)))
+            role = find_role(ROLE_RC, L);
+        if (role) inst = &role->inst;
+        st.rc = role && role->role == ROLE_RC;
         if (!inst) throw SipError(AsdSip::ACL_ERROR_API_NOT_SUPPORT, "no kernel for length " + std::to_string(L));
         st.kind = StageKind::Stockham;
         st.in = in.buf;
@@ -499,7 +515,8 @@ struct Builder {
         a.LP = lp;
         const int T = inst->T;
         const bool column = a.tin.unit_f || a.tout.unit_f;
-        const size_t per = ci ? (size_t)lp * 4 : (size_t)2 * lp * 4 + 24;
+        const bool one_plane = role && role->role != ROLE_RC && role->role != ROLE_REAL_ROWS;
+        const size_t per = one_plane ? (size_t)lp * 4 : (size_t)2 * lp * 4 + 24;
         int F;
         if (column) {
             // Tile width: a multiple of 16 transforms (each row run covers whole 128-byte lines),
@@ -517,12 +534,12 @@ struct Builder {
             // A tile of one wave or less takes a whole one (20 x 419430, one thread per column: 34 us at
             // 16 wide, 22 us at 64).
             const bool pow2 = (L & (L - 1)) == 0;
-            if (want <= 0 && ci) want = ci->F;
+            if (want <= 0 && role) want = role->F;
             F = want > 0 ? want : pow2 ? std::min(64, std::max(16, (512 / T) & ~15)) : T >= 4 ? 16 : T >= 2 ? 32 : 64;
             if (F >= 16) F &= ~15;
             while (F > 1 && ((size_t)F * per > 160 * 1024 || F * T > 1024)) F /= 2;
         } else {
-            F = std::max(1, 256 / T);
+            F = role && role->F ? role->F : std::max(1, 256 / T);
             while (F > 1 && ((size_t)F * per > 48 * 1024 || F * T > 1024)) F--;
             int f = p.tune.row_F;
             if (f <= 0) {
@@ -567,9 +584,9 @@ struct Builder {
         // First / last radix pass straight from / to HBM for contiguous complex rows, when a
         // transform has enough threads for its accesses to coalesce.
         a.direct_in = (io_mode == IO_C2C || io_mode == IO_R2C_EVEN) && a.tin.es == 1 && !a.tin.unit_f &&
-                      (T >= 16 || mf != nullptr);
+                      (T >= 16 || mf != nullptr || (role && role->role == ROLE_ROWS));
         a.direct_out = (io_mode == IO_C2C || io_mode == IO_C2R_EVEN) && a.tout.es == 1 && !a.tout.unit_f &&
-                       (T >= 16 || mf != nullptr) && tw4_ntot == 0;
+                       (T >= 16 || mf != nullptr || (role && role->role == ROLE_ROWS)) && tw4_ntot == 0;
         // split-plane user buffers go through the LDS-staged load / store
         a.in_sep = in_sep ? 1 : 0;
         a.out_sep = out_sep ? 1 : 0;
@@ -581,53 +598,23 @@ struct Builder {
             a.direct_out = 0;
             a.tout.vec2 = 0;
         }
-        const bool rows = io_mode == IO_C2C && a.direct_in && a.direct_out && inst->rows_fwd != nullptr;
         a.col_direct = columns && (!mf || mf_cols) ? 1 : 0;
-        // Single-plane exchange (half the LDS, twice the resident workgroups) by default for rows
-        // with 32 or more threads per transform. Measured on MI355X, 1 GiB of C2C rows: 4096
-        // 373 us against 397 us, 1024 370 / 395, 8192 428 / 497, 16384 436 / 646; at 16 threads
-        // (length 256) the two-plane kernel stays ahead (371 / 381). Launch order beats
-        // XCD-contiguous tile order (4096 x 16384: 0.194 against 0.200 ms); the latter stays
-        // available as the tuning switch SIP_FFT_XCD=1.
-        a.split_lds = rows && (p.tune.split_lds >= 0 ? p.tune.split_lds == 1
-                                                     : env_flag("SIP_FFT_SPLIT_LDS", T >= 32 || mf != nullptr));
-        if (L > kRowLeafMax) {
-            // single-pass leaves above 16384 exist only as the single-plane rows kernel
-            if (!rows)
-                throw SipError(AsdSip::ACL_ERROR_INTERNAL_ERROR, "length " + std::to_string(L) + " leaf off contiguous rows");
-            a.split_lds = 1;
-        }
-        // Column tiles with direct HBM passes: single plane too (a 1024 x 16 tile needs 70 KiB
-        // instead of 139 KiB, so two workgroups fit on a CU). Measured on MI355X: 2D 1024^2 x 128
-        // 892 -> 863 us, 1024^2 x 8 52 -> 48 us, 512^2 x 256 445 -> 422 us, 2^20 x 64 606 -> 566 us;
-        // with 16-wide mixed-length tiles and the derived four-step twiddles, mixed lengths gain
-        // too: four-step 43200 x 1056 387-399 -> 346 us, 64000 x 635 370 -> 337 us, 2D 1000^2 x 64
-        // 528-535 -> 500 us, 3D 240^3 x 8 1155 -> 1086 us.
-        if (a.col_direct && (ci || (mf && split_columns(L)))) a.split_lds = 1;
-        // Fused real transforms on contiguous rows: single plane as well (pair pre-process read
-        // straight from HBM for C2R, post-process through the plane for R2C). Measured on MI355X:
-        // 8192 x 4096 R2C 58.1 -> 47.5 us, C2R 58.8 -> 46.7 us; 12000 x 2048 77 / 82 -> 68 / 67 us;
-        // 2000 x 8192 40 / 38 -> 36 / 34 us; 3000 and 6000 R2C unchanged.
-        const bool real_rows = (io_mode == IO_R2C_EVEN && a.direct_in && a.tout.es == 1 && !a.tout.unit_f) ||
-                               (io_mode == IO_C2R_EVEN && a.direct_out && a.tin.es == 1 && !a.tin.unit_f);
-        if (real_rows && inst->real_rows[0] != nullptr && env_flag("SIP_FFT_SPLIT_REAL", true)) a.split_lds = 1;
-        // Rows in, columns out (the second four-step stage: contiguous rows of the intermediate,
-        // transposed store): one plane, the first pass straight from HBM along each row, the last
-        // pass straight to HBM across adjacent transforms (instead of the two-plane tile with
-        // LDS-staged store).
-        st.rc = io_mode == IO_C2C && !mf && !in_sep && !out_sep && a.tin.es == 1 && !a.tin.unit_f &&
-                a.tout.unit_f && tw4_ntot == 0 && inst->rc[0] != nullptr &&
-                (p.tune.rc >= 0 ? p.tune.rc == 1 : env_flag("SIP_FFT_RC", true));
-        if (st.rc) {
-            a.split_lds = 0;
-            a.col_direct = 0;
-        }
+        // Single-plane exchange (half the LDS, twice the resident workgroups) wherever a role has it, and
+        // for the matrix-core rows and column tiles. Measured on MI355X, 1 GiB of C2C rows, one / two planes:
+        // 4096 373 / 397 us, 1024 370 / 395, 8192 428 / 497, 16384 436 / 646; 2D 1024^2 x 128 863 / 892;
+        // R2C 8192 x 4096 47.5 / 58.1, C2R 46.7 / 58.8.
+        if (L > kRowLeafMax && !(role && role->role == ROLE_ROWS))
+            throw SipError(AsdSip::ACL_ERROR_INTERNAL_ERROR, "length " + std::to_string(L) + " leaf off contiguous rows");
+        const bool mf_rows = mf && flat_in && flat_out && tw4_ntot == 0 && inst->rows_fwd != nullptr &&
+                             (p.tune.split_lds >= 0 ? p.tune.split_lds == 1 : env_flag("SIP_FFT_SPLIT_LDS", true));
+        a.split_lds = ((role && !st.rc) || mf_rows || (mf && a.col_direct && split_columns(L))) ? 1 : 0;
+        if (st.rc) a.col_direct = 0;
         // Workgroups go round robin to the 8 XCDs, each with its own L2. Where a column tile's runs do not
         // start on 128-byte lines (a stride that is not a multiple of 16 elements), adjacent tiles share
         // lines, which two L2s would fetch and write apart: XCD-contiguous tile order. Measured on
         // MI355X, launch / XCD-contiguous order, columns of 64 MiB: 100 x 83886 35.2 / 26.7 us, 243 x
         // 34521 38.9 / 28.1, 1080 x 7767 42.4 / 36.8, R2C 512^2 x 64 68.9 / 54.9; whole lines lose by it:
-        // 256 x 32768 22.8 / 25.0, 1024 x 8192 25.8 / 27.9.
+        // 256 x 32768 22.8 / 25.0, 1024 x 8192 25.8 / 27.9; so do rows (4096 x 16384 0.194 / 0.200 ms).
         const bool split_lines = (a.tin.unit_f && a.tin.es % 16 != 0) || (a.tout.unit_f && a.tout.es % 16 != 0);
         a.xcd_remap = p.tune.xcd >= 0 ? p.tune.xcd == 1 : env_flag("SIP_FFT_XCD", column && split_lines);
         // matrix passes read [k][16] twiddle rows; the single-plane rows kernel (K = 32) reads the

@@ -186,8 +186,8 @@ std::string plan_describe(const Plan &p);
 
 // Kernel registry (generated instances).
 const StockhamInstance *find_instance(int64_t L);
-// Column-tile kernels of a length, with or without the four-step twiddle, or null.
-const ColumnInstance *find_column_instance(int64_t L, bool tw4);
+// Single-plane kernels of a role and length, or null.
+const RoleInstance *find_role(Role role, int64_t L);
 // Split-precision MFMA instances (mode = PrecisionMode) and their DFT-matrix operand table.
 const StockhamInstance *find_mfma_instance(int64_t L, int mode);
 // Fused 2D tile instance for X x Y slices (X, Y in 32, 64, 128), or null.

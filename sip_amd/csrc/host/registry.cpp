@@ -62,24 +62,23 @@ const BluesteinInstance *find_bluestein_instance(int64_t min_m)
     return nullptr;
 }
 
-#define SIP_COLUMNS_PART(k)                              \
-    extern const ColumnInstance g_columns_part_##k[];    \
-    extern const int g_columns_part_##k##_count;
-#include "columns_parts.inc"
-#undef SIP_COLUMNS_PART
+#define SIP_ROLE_PART(name)                   \
+    extern const RoleInstance g_##name[];     \
+    extern const int g_##name##_count;
+#include "role_parts.inc"
+#undef SIP_ROLE_PART
 
-const ColumnInstance *find_column_instance(int64_t L, bool tw4)
+const RoleInstance *find_role(Role role, int64_t L)
 {
     static const auto m = [] {
-        std::map<std::pair<int64_t, bool>, const ColumnInstance *> r;
-#define SIP_COLUMNS_PART(k)                                         \
-    for (int i = 0; i < g_columns_part_##k##_count; i++)            \
-        r[{g_columns_part_##k[i].inst.L, g_columns_part_##k[i].inst.cols[2] != nullptr}] = &g_columns_part_##k[i];
-#include "columns_parts.inc"
-#undef SIP_COLUMNS_PART
+        std::map<std::pair<int, int64_t>, const RoleInstance *> r;
+#define SIP_ROLE_PART(name) \
+    for (int i = 0; i < g_##name##_count; i++) r[{g_##name[i].role, g_##name[i].inst.L}] = &g_##name[i];
+#include "role_parts.inc"
+#undef SIP_ROLE_PART
         return r;
     }();
-    auto it = m.find({L, tw4});
+    auto it = m.find({role, L});
     return it == m.end() ? nullptr : it->second;
 }
 

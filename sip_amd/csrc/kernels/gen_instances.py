@@ -16,6 +16,7 @@ import sys
 
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))  # also when loaded from a path
 from column_shapes import COLUMN_SHAPES, COLUMN_TW_SHAPES, LONG_COLUMN_SHAPES
+from row_shapes import ROW_SHAPES
 
 MAX_SMOOTH = 16384
 MAX_POW2 = 16384
@@ -59,7 +60,7 @@ def factor(n):
 # alternative was faster by more than 5 % (run-to-run spread: median 0.6 %, at most 3.4 % in the
 # first round, 6.2 % in the second, whose kept gains are all above 10 %). Old / new microseconds in
 # the comments.
-SEQ_OVERRIDE = {
+LEAF_SEQ = {
     1120: [16, 10, 7],       # 51.6 / 46.6
     1200: [20, 12, 5],       # 49.6 / 46.6
     1280: [16, 10, 8],       # 46.0 / 40.9
@@ -98,6 +99,8 @@ SEQ_OVERRIDE = {
     25920: [16, 9, 9, 5, 4],  # 206 / 193
     30000: [10, 10, 10, 6, 5],  # 258 / 215
 }
+# The sequences these lengths run as contiguous rows: the row kernel's own where one was measured faster.
+SEQ_OVERRIDE = {n: ROW_SHAPES[n][1] if n in ROW_SHAPES else seq for n, seq in LEAF_SEQ.items()}
 # (1000 = 10 x 10 x 10 was faster in the four-step roles, 305 / 283 us, but its 100 threads per
 # transform halve the column tiles to 8 transforms, half-line HBM runs: 2D 1000^2 gained nothing.)
 
@@ -140,8 +143,8 @@ def radix_sequence(n):
     radices <= 16. Other lengths: the sequence over RADICES (composites included) with the lowest
     _cost, ties to the larger leading radices. Largest radices first."""
     if n & (n - 1):
-        if n in SEQ_OVERRIDE:
-            return list(SEQ_OVERRIDE[n])
+        if n in LEAF_SEQ:
+            return list(LEAF_SEQ[n])
         ranked = []
         for seq in _sequences(n):
             c = _cost(n, seq)
@@ -223,8 +226,8 @@ def big_threads(n, seq):
 def big_radix_sequence(n):
     """Fewest passes over BIG_RADICES within BIG_MAX_ELEMS values per thread, then the fewest idle
     butterfly rounds; largest radices first."""
-    if n in SEQ_OVERRIDE:
-        return list(SEQ_OVERRIDE[n])
+    if n in LEAF_SEQ:
+        return list(LEAF_SEQ[n])
     found = []
 
     def rec(m, maxr, seq):
@@ -270,53 +273,16 @@ def instances():
     return res
 
 
-# Lengths whose contiguous C2C rows run faster on the two-plane tile than on the single-plane rows
-# kernel (no rows kernel is emitted for them, so the planner and the tuner keep the tile). Measured
-# on MI355X, 256 MiB of rows, single / two planes: 12000 208 / 179 us, 15000 189 / 164, 15625
-# 288 / 240, 16200 233 / 201, 14580 190 / 168, 12150 205 / 181, 8748 141 / 134, 12960 173 / 164,
-# 15552 169 / 158; every other length from 4320 to 16384 is faster on one plane (up to 1.7x).
-ROWS_TWO_PLANE = {8748, 12000, 12150, 12960, 14580, 15000, 15552, 15625, 16200}
+# Contiguous-row kernels (rows.h) from ROWS_MIN points up, with three or more threads per transform: shorter
+# rows, and leaves of fewer threads, are faster staged through LDS in line order (16: 5.3-6.0 TB/s staged,
+# 4.1 from their own threads). Two lengths are faster on the two-plane tile: 256 MiB of rows, single / two
+# planes, 15625 268 / 240 us, 15552 171 / 158.
+ROWS_MIN, ROWS_MIN_THREADS = 24, 3
+ROWS_TWO_PLANE = {15552, 15625}
 
 # longest leaf used for column tiles (the host's kColumnLeafMax); every leaf up to it gets a column
 # kernel of its own (columns.h) with the shape measured for that role (column_shapes.py)
 COLUMN_LEAF_MAX = 1024
-COLUMN_PARTS = 16
-def column_instances():
-    """(length, four-step twiddle, threads, radices, waves per SIMD or 0, columns per tile or 0 for the
-    planner's rule)."""
-    out = []
-    for n, t, seq in instances():
-        if n <= COLUMN_LEAF_MAX:
-            for tw, shapes in ((False, COLUMN_SHAPES), (True, COLUMN_TW_SHAPES)):
-                out.append((n, tw) + tuple(shapes.get(n, (t, seq, 0))) + (0,))
-    out += [(n, False) + shape for n, shape in LONG_COLUMN_SHAPES.items()]
-    for n, _, t, seq, _, f in out:
-        p = 1
-        for r in seq:
-            p *= r
-        assert p == n and elems_per_thread(n, seq, t) <= 40 and (f or 1) * t <= 1024, (n, t, seq)
-    return sorted(out)
-
-
-def write_columns(outdir):
-    inst = column_instances()
-    for k in range(COLUMN_PARTS):
-        items = inst[k::COLUMN_PARTS]
-        lines = ["// Generated by gen_instances.py: column-tile kernels (do not edit).", '#include "columns.h"',
-                 "namespace sip {", f"extern const ColumnInstance g_columns_part_{k}[] = {{"]
-        for n, tw, t, seq, w, f in items:
-            rs = ", ".join(str(r) for r in seq)
-            names = [f"(const void *)&stockham_cols_kernel<{w}, {n}, {t}, {sg}, {str(tw).lower()}, {rs}>"
-                     for sg in (-1, 1)]
-            cols = ", ".join(["nullptr, nullptr"] * tw + names + ["nullptr, nullptr"] * (not tw))
-            lines.append(f"    {{{{{n}, {t}, {len(seq)}, {{{rs}}}, nullptr, nullptr, nullptr, nullptr, "
-                         f"{{{cols}}}, {{nullptr, nullptr, nullptr, nullptr}}, {{nullptr, nullptr}}}}, {f}}},")
-        lines += ["};", f"extern const int g_columns_part_{k}_count = {len(items)};", "}  // namespace sip"]
-        write_if_changed(os.path.join(outdir, f"columns_part_{k}.hip"), "\n".join(lines) + "\n")
-    inc = ["// Generated by gen_instances.py (do not edit)."] + [f"SIP_COLUMNS_PART({k})" for k in range(COLUMN_PARTS)]
-    write_if_changed(os.path.join(outdir, "columns_parts.inc"), "\n".join(inc) + "\n")
-
-
 # half lengths (with 32 or more threads per transform) of the real transforms that also get
 # single-plane R2C / C2R row kernels: every one up to 8192, and those above 8192 where the single
 # plane measured faster than the two-plane fused kernel on MI355X (R2C + C2R of 256 MiB of reals,
@@ -329,6 +295,77 @@ REAL_ROWS_LONG = {8640, 9000, 9216, 9375, 9600, 9720, 10000, 10125, 10240, 10368
 # transform (64-byte runs per row read) also get the rows-in / columns-out kernel of the second
 # four-step stage
 RC_MIN_THREADS = 8
+
+
+def role_entry(role, n, t, seq, f, slot, names):
+    """A RoleInstance initialiser whose kernels fill `slot` of the instance."""
+    slots = {"tile": "nullptr, nullptr", "rows": "nullptr, nullptr", "cols": "{nullptr, nullptr, nullptr, nullptr}",
+             "real": "{nullptr, nullptr, nullptr, nullptr}", "rc": "{nullptr, nullptr}"}
+    names = ", ".join(nm if nm == "nullptr" else f"(const void *)&{nm}" for nm in names)
+    slots[slot] = names if slot == "rows" else "{" + names + "}"
+    p = 1
+    for r in seq:
+        p *= r
+    assert p == n and elems_per_thread(n, seq, t) <= 40 and (f or 1) * t <= 1024, (n, t, seq)
+    rs = ", ".join(str(r) for r in seq)
+    return f"    {{{role}, {f}, {{{n}, {t}, {len(seq)}, {{{rs}}}, {', '.join(slots.values())}}}}},"
+
+
+def row_entries():
+    for n, t, seq in instances():
+        t, seq, w, f = ROW_SHAPES.get(n, (t, seq, 0, 0))
+        if n < ROWS_MIN or t < ROWS_MIN_THREADS or n in ROWS_TWO_PLANE:
+            continue
+        rs = ", ".join(str(r) for r in seq)
+        yield role_entry("ROLE_ROWS", n, t, seq, f, "rows", [f"stockham_rows_kernel<{w}, {n}, {t}, {sg}, {rs}>" for sg in (-1, 1)])
+
+
+def real_row_entries():
+    for n, t, seq in instances():
+        if n <= MAX_SMOOTH and t >= 32 and (n <= REAL_ROWS_MAX or n in REAL_ROWS_LONG):
+            rs = ", ".join(str(r) for r in seq)
+            yield role_entry("ROLE_REAL_ROWS", n, t, seq, 0, "real", [
+                f"stockham_real_rows_kernel<{n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)])
+
+
+def column_entries():
+    shapes = []
+    for n, t, seq in instances():
+        if n <= COLUMN_LEAF_MAX:
+            shapes.append((n, False) + tuple(COLUMN_SHAPES.get(n, (t, seq, 0))) + (0,))
+            shapes.append((n, True) + tuple(COLUMN_TW_SHAPES.get(n, (t, seq, 0))) + (0,))
+    shapes += [(n, False) + shape for n, shape in LONG_COLUMN_SHAPES.items()]
+    for n, tw, t, seq, w, f in shapes:
+        rs = ", ".join(str(r) for r in seq)
+        names = [f"stockham_cols_kernel<{w}, {n}, {t}, {sg}, {str(tw).lower()}, {rs}>" for sg in (-1, 1)]
+        none = ["nullptr", "nullptr"]
+        yield role_entry("ROLE_COLS_TW" if tw else "ROLE_COLS", n, t, seq, f, "cols", none + names if tw else names + none)
+
+
+def rc_entries():
+    for n, t, seq in instances():
+        if n <= COLUMN_LEAF_MAX and len(seq) >= 2 and t >= RC_MIN_THREADS:
+            rs = ", ".join(str(r) for r in seq)
+            yield role_entry("ROLE_RC", n, t, seq, 0, "rc", [f"stockham_rc_kernel<{n}, {t}, {sg}, {rs}>" for sg in (-1, 1)])
+
+
+# role files: name, header, entries, parts
+ROLE_FILES = [("rows", "rows.h", row_entries, 16), ("real_rows", "real_rows.h", real_row_entries, 16),
+              ("columns", "columns.h", column_entries, 16), ("rows_cols", "rows_cols.h", rc_entries, 8)]
+
+
+def write_roles(outdir):
+    inc = ["// Generated by gen_instances.py (do not edit)."]
+    for name, header, entries, parts in ROLE_FILES:
+        items = list(entries())
+        for k in range(parts):
+            part = items[k::parts]
+            text = ["// Generated by gen_instances.py (do not edit).", f'#include "{header}"', "namespace sip {",
+                    f"extern const RoleInstance g_{name}_part_{k}[] = {{"] + part
+            text += ["};", f"extern const int g_{name}_part_{k}_count = {len(part)};", "}  // namespace sip"]
+            write_if_changed(os.path.join(outdir, f"{name}_part_{k}.hip"), "\n".join(text) + "\n")
+            inc.append(f"SIP_ROLE_PART({name}_part_{k})")
+    write_if_changed(os.path.join(outdir, "role_parts.inc"), "\n".join(inc) + "\n")
 
 
 # One-launch inverse short-time transforms (istft.h): every 2,3,5-smooth frame length in this range,
@@ -367,8 +404,8 @@ def main():
     nparts = int(sys.argv[2])
     os.makedirs(outdir, exist_ok=True)
     write_istft(outdir)
-    write_columns(outdir)
-    inst = instances()
+    write_roles(outdir)
+    inst = [i for i in instances() if i[0] <= MAX_SMOOTH]  # longer leaves are row kernels only
     parts = [[] for _ in range(nparts)]
     # balance by estimated code size (passes x length)
     load = [0] * nparts
@@ -387,44 +424,12 @@ def main():
         for n, t, seq in items:
             rs = ", ".join(str(r) for r in seq)
             radix = ", ".join(str(r) for r in seq)
-            if n > MAX_SMOOTH:
-                rf = f"stockham_rows_kernel<{n}, {t}, -1, {rs}>"
-                ri = f"stockham_rows_kernel<{n}, {t}, 1, {rs}>"
-                lines.append(f"template __global__ void {rf}(const StockhamArgs);")
-                lines.append(f"template __global__ void {ri}(const StockhamArgs);")
-                tab.append(f"    {{{n}, {t}, {len(seq)}, {{{radix}}}, nullptr, nullptr, (const void *)&{rf}, "
-                           f"(const void *)&{ri}, {{nullptr, nullptr, nullptr, nullptr}}, "
-                           f"{{nullptr, nullptr, nullptr, nullptr}}, {{nullptr, nullptr}}}},")
-                continue
             kf = f"stockham_kernel<{n}, {t}, -1, {rs}>"
             ki = f"stockham_kernel<{n}, {t}, 1, {rs}>"
             lines.append(f"template __global__ void {kf}(const StockhamArgs);")
             lines.append(f"template __global__ void {ki}(const StockhamArgs);")
-            if t >= 16 and n not in ROWS_TWO_PLANE:
-                rf = f"stockham_rows_kernel<{n}, {t}, -1, {rs}>"
-                ri = f"stockham_rows_kernel<{n}, {t}, 1, {rs}>"
-                lines.append(f"template __global__ void {rf}(const StockhamArgs);")
-                lines.append(f"template __global__ void {ri}(const StockhamArgs);")
-                rows = f"(const void *)&{rf}, (const void *)&{ri}"
-            else:
-                rows = "nullptr, nullptr"
-            if t >= 32 and (n <= REAL_ROWS_MAX or n in REAL_ROWS_LONG):
-                names = [f"stockham_real_rows_kernel<{n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)]
-                for nm in names:
-                    lines.append(f"template __global__ void {nm}(const StockhamArgs);")
-                real = "{" + ", ".join(f"(const void *)&{nm}" for nm in names) + "}"
-            else:
-                real = "{nullptr, nullptr, nullptr, nullptr}"
-            if n <= COLUMN_LEAF_MAX and len(seq) >= 2 and t >= RC_MIN_THREADS:
-                names = [f"stockham_rc_kernel<{n}, {t}, {sg}, {rs}>" for sg in (-1, 1)]
-                for nm in names:
-                    lines.append(f"template __global__ void {nm}(const StockhamArgs);")
-                rc = "{" + ", ".join(f"(const void *)&{nm}" for nm in names) + "}"
-            else:
-                rc = "{nullptr, nullptr}"
-            tab.append(f"    {{{n}, {t}, {len(seq)}, {{{radix}}}, (const void *)&{kf}, (const void *)&{ki}, {rows}, "
-                       "{nullptr, nullptr, nullptr, nullptr}, "
-                       f"{real}, {rc}}},")
+            tab.append(f"    {{{n}, {t}, {len(seq)}, {{{radix}}}, (const void *)&{kf}, (const void *)&{ki}, nullptr, nullptr, "
+                       "{nullptr, nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr, nullptr}, {nullptr, nullptr}},")
         lines.append(f"extern const StockhamInstance g_stockham_part_{k}[] = {{")
         lines += tab
         lines.append("};")

@@ -95,31 +95,38 @@ enum PrecisionMode : int32_t {
     PREC_BF16_SPLIT3 = 3 // MFMA, BF16 hi+mid+lo operands
 };
 
-// Host-side view of one compiled kernel instance.
-typedef void (*StockhamKernelFn)(StockhamArgs);
+// Host-side view of one compiled kernel instance: a length's threads, radix sequence and kernels
+// (__global__ function handles, hipLaunchKernel symbols; forward / inverse, null where there are none).
+// Every leaf length has a generic tile instance (fwd / inv). The single-plane kernels of one role have
+// instances of their own, with the threads and radices measured for it (RoleInstance).
 struct StockhamInstance {
     int32_t L;
     int32_t T;               // threads per transform
     int32_t npass;
     int32_t radix[12];
-    const void *fwd;         // __global__ function handles (hipLaunchKernel symbol)
+    const void *fwd;         // generic two-plane tile
     const void *inv;
-    const void *rows_fwd;    // single-plane contiguous-row kernels (T >= 16 only, else null)
+    const void *rows_fwd;    // contiguous rows
     const void *rows_inv;
-    const void *cols[4];     // single-plane column-tile kernels, fwd / inv without and fwd / inv
-                             // with the four-step twiddle (column and matrix-core instances only)
-    const void *real_rows[4];  // single-plane R2C fwd / inv, C2R fwd / inv rows (T >= 32; L <= 8192
-                               // and the longer L where they measured faster; else null)
-    const void *rc[2];         // single-plane rows-in / columns-out fwd / inv (four-step second
-                               // stage; L <= 1024 with two or more passes and T >= 8, else null)
+    const void *cols[4];     // column tiles, fwd / inv without and fwd / inv with the four-step twiddle
+    const void *real_rows[4];  // R2C fwd / inv, C2R fwd / inv rows
+    const void *rc[2];         // rows in, columns out (four-step second stage)
 };
 
-// Column-tile kernels of one length, with the threads and radices measured for that role: `inst` holds
-// L, T, the radices and cols[] only. The kernels with the four-step twiddle on store have an entry of
-// their own (cols[2..3]; lengths up to 1024), those without another (cols[0..1]; up to 4096).
-struct ColumnInstance {
+// Roles of the single-plane kernels.
+enum Role : int32_t {
+    ROLE_ROWS = 0,       // contiguous C2C rows (rows.h)
+    ROLE_REAL_ROWS = 1,  // contiguous R2C / C2R rows of half length L (real_rows.h)
+    ROLE_COLS = 2,       // column tiles (columns.h)
+    ROLE_COLS_TW = 3,    // column tiles with the four-step twiddle on store
+    ROLE_RC = 4,         // rows in, columns out (rows_cols.h)
+    ROLE_PLANES = 5      // contiguous rows in two planes (planes.h); one direction, in rows_fwd
+};
+
+struct RoleInstance {
+    int32_t role;
+    int32_t F;  // transforms per workgroup; 0 = the planner's rule
     StockhamInstance inst;
-    int32_t F;  // columns per tile; 0 = the planner's rule
 };
 
 // Registry entry of a fused 2D tile instance (stockham2d.h). The radix sequences, and so the

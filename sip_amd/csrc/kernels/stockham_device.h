@@ -612,26 +612,6 @@ __device__ __forceinline__ int64_t tile_index(const StockhamArgs &a)
     return tile;
 }
 
-// Contiguous C2C rows, single LDS plane (separate kernel so that its register budget is its own).
-template <int L, int T, int S, int... Rs>
-__global__ __launch_bounds__(1024) void stockham_rows_kernel(const StockhamArgs a)
-{
-    extern __shared__ float lds[];
-    split_rows<L, T, S, false, Rs...>(a, lds, tile_index(a));
-}
-
-// Real-transform rows, single LDS plane: MODE 1 = R2C (half-length C2C + pair post-process),
-// MODE 2 = C2R (pair pre-process + half-length C2C).
-template <int L, int T, int S, int MODE, int... Rs>
-__global__ __launch_bounds__(1024) void stockham_real_rows_kernel(const StockhamArgs a)
-{
-    extern __shared__ float lds[];
-    if constexpr (MODE == 1)
-        split_rows<L, T, S, true, Rs...>(a, lds, tile_index(a));
-    else
-        split_rows_c2r<L, T, S, Rs...>(a, lds, tile_index(a));
-}
-
 // Strided transform of a column tile: element j at in[j * es_in] / out[j * es_out], with the
 // four-step twiddle W^{col * j} applied on store when the stage carries one. TW: 0 = the stage has
 // no four-step twiddle, 1 = it has one, 2 = decided at run time (tw4_ntot). The single-plane
@@ -777,13 +757,6 @@ __device__ __forceinline__ void split_rows_cols(const StockhamArgs &a, float *pl
     }
     const ColIoT<0> io{nullptr, static_cast<float2 *>(a.out) + ob, 0, a.tout.es, 0, &a};
     split_chain<L, T, S, 1, R0, Rest...>(pl, a.tw, fr * a.LP, tr, act1, v, io, LastRemap{fc * a.LP, tc, act2});
-}
-
-template <int L, int T, int S, int... Rs>
-__global__ __launch_bounds__(1024) void stockham_rc_kernel(const StockhamArgs a)
-{
-    extern __shared__ float lds[];
-    split_rows_cols<L, T, S, Rs...>(a, lds, tile_index(a));
 }
 
 // Pass runners: the radix chain the tile goes through between load and store.

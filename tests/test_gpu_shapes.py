@@ -74,3 +74,21 @@ def test_streaming_input_of_several_launches(torch_cuda):
     h = make([1 << 20], S.ASCEND_FFT_C2C, FWD, 5)
     assert [s["nt_in"] for s in h.describe()["stages"]] == [0, 0]
     h.destroy()
+
+
+ROWS = _shapes("row_shapes")
+
+
+@pytest.mark.parametrize("n", sorted(ROWS.ROW_SHAPES) + [25, 27, 35, 64, 66, 104, 117, 128, 16200])
+def test_row_shapes(torch_cuda, n):
+    b = max(3, min(75, (1 << 19) // n))
+    d = INV if n % 3 else FWD
+    h = make([n], S.ASCEND_FFT_C2C, d, b)
+    st = h.describe()["stages"][0]
+    h.destroy()
+    assert st["split_lds"] == st["direct_in"] == st["direct_out"] == 1
+    if n in ROWS.ROW_SHAPES:
+        assert st["T"] == ROWS.ROW_SHAPES[n][0] and st["radices"] == ROWS.ROW_SHAPES[n][1]
+    x = oracle.uniform_complex((b, n), 0x5EED1000 + n)
+    rel, _ = report(f"rows {n} x {b}", c2c(x, [n], d), oracle.c2c(x, sign_of(d)))
+    assert rel <= TOL
