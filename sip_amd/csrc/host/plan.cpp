@@ -439,6 +439,12 @@ struct Builder {
     // passes, from 128 tiles up (half of the CUs). Measured on MI355X, two passes / one, 64 MiB of columns:
     // 1080 60 / 35 us, 2048 56 / 30, 4096 54 / 42; fewer tiles leave the chip to a few long workgroups: 2048
     // x 100 columns (7 tiles) 9 / 19 us, R2C 1080 x 1920 (61 tiles) 26 / 28 us, C2C 2048 x 2048 (128) 44 / 37.
+    // Contiguous transforms of length L, each starting where the one before ends
+    static bool whole_rows(const TileDesc &t, int64_t L)
+    {
+        return t.es == 1 && t.tab_dim < 0 && t.n1 == 1 && (t.n0 == 1 || t.s0 == L);
+    }
+
     bool long_columns(int64_t L, const Lay &in, const Lay &out) const
     {
         const RoleInstance *ci = L > kColumnLeafMax ? find_role(ROLE_COLS, L) : nullptr;
@@ -487,6 +493,11 @@ struct Builder {
         else if (io_mode == IO_C2C && !mf && flat_in && tout.unit_f && !out_sep && tw4_ntot == 0 &&
                  (p.tune.rc >= 0 ? p.tune.rc == 1 : env_flag("SIP_FFT_RC", true)))
             role = find_role(ROLE_RC, L);
+        // Split planes on both sides, rows one after the other (the kernel of up to 48 points reads them as one run)
+        else if (io_mode == IO_C2C && in_sep && out_sep && tw4_ntot == 0 && whole_rows(tin, L) && whole_rows(tout, L) &&
+                 env_flag("SIP_FFT_SPLIT_LDS", true))
+            role = find_role(ROLE_PLANES, L);
+        st.planes = role && role->role == ROLE_PLANES;
         if (role) inst = &role->inst;
         st.rc = role && role->role == ROLE_RC;
         if (!inst) throw SipError(AsdSip::ACL_ERROR_API_NOT_SUPPORT, "no kernel for length " + std::to_string(L));
@@ -620,7 +631,7 @@ struct Builder {
         // matrix passes read [k][16] twiddle rows; the single-plane rows kernel (K = 32) reads the
         // interleaved operand table, the two-plane tile (K = 16) the blocked one
         const bool mf2 = mf != nullptr && a.split_lds;
-        st.tw = pass_twiddles(inst, sign, mf != nullptr);
+        st.tw = pass_twiddles(inst, st.planes ? -1 : sign, mf != nullptr);
         if (mf) st.mfw = mf2 ? mfma2_dft_table(p.precision, sign) : mfma_dft_table(p.precision, sign);
         if (io_mode == IO_R2C_EVEN || io_mode == IO_C2R_EVEN) st.rtw = real_roots(L, sign);
         if (tw4_ntot) {
@@ -1262,6 +1273,7 @@ static const void *stage_kernel(const Stage &s)
     if (s.sa.split_lds && s.sa.col_direct) return s.inst->cols[(s.sa.tw4_ntot != 0 ? 2 : 0) + (s.sign < 0 ? 0 : 1)];
     if (s.sa.split_lds && s.sa.io_mode == IO_R2C_EVEN) return s.inst->real_rows[s.sign < 0 ? 0 : 1];
     if (s.sa.split_lds && s.sa.io_mode == IO_C2R_EVEN) return s.inst->real_rows[s.sign < 0 ? 2 : 3];
+    if (s.planes) return s.inst->rows_fwd;
     if (s.sa.split_lds) return s.sign < 0 ? s.inst->rows_fwd : s.inst->rows_inv;
     return s.sign < 0 ? s.inst->fwd : s.inst->inv;
 }
@@ -1477,6 +1489,14 @@ void plan_execute_sep(Plan &p, const void *in, const void *in_im, void *out, voi
             a.out_im = im_of(s.out);
             if ((a.in_sep && !a.in_im) || (a.out_sep && !a.out_im))
                 throw SipError(AsdSip::ACL_ERROR_INTERNAL_ERROR, "split-plane plan executed without imaginary planes");
+            if (s.planes && s.sign > 0) {
+                const void *re = a.in;
+                a.in = a.in_im;
+                a.in_im = static_cast<const float *>(re);
+                void *ore = a.out;
+                a.out = a.out_im;
+                a.out_im = static_cast<float *>(ore);
+            }
             if (a.tin.vec2 && (reinterpret_cast<uintptr_t>(src) & 15)) a.tin.vec2 = 0;
             if (a.tout.vec2 && (reinterpret_cast<uintptr_t>(dst) & 15)) a.tout.vec2 = 0;
             void *args[] = {&a};

@@ -86,6 +86,8 @@ struct Stage {
     TableRef tw2;
     // rows-in / columns-out kernel (four-step second stage: contiguous rows, transposed store)
     bool rc = false;
+    // split-plane rows kernel (forward; an inverse stage swaps the planes on both sides)
+    bool planes = false;
     int in_tab = -1, out_tab = -1;  // row tables (Plan::row_tables) gathered by the in / out side
     // Aux
     AuxArgs xa{};

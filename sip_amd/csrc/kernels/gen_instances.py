@@ -320,6 +320,22 @@ def row_entries():
         yield role_entry("ROLE_ROWS", n, t, seq, f, "rows", [f"stockham_rows_kernel<{w}, {n}, {t}, {sg}, {rs}>" for sg in (-1, 1)])
 
 
+# Split-plane rows up to this length go through LDS in line order (planes.h)
+PLANES_SMALL_MAX = 48
+
+
+def plane_entries():
+    for n, t, seq in instances():
+        if n > MAX_SMOOTH:
+            continue
+        w, f = 0, 0
+        if n > PLANES_SMALL_MAX:
+            t, seq, w, f = ROW_SHAPES.get(n, (t, seq, 0, 0))
+        rs = ", ".join(str(r) for r in seq)
+        name = f"planes_small_kernel<{n}, {t}, {rs}>" if n <= PLANES_SMALL_MAX else f"planes_rows_kernel<{w}, {n}, {t}, {rs}>"
+        yield role_entry("ROLE_PLANES", n, t, seq, f, "rows", [name, "nullptr"])
+
+
 def real_row_entries():
     for n, t, seq in instances():
         if n <= MAX_SMOOTH and t >= 32 and (n <= REAL_ROWS_MAX or n in REAL_ROWS_LONG):
@@ -351,7 +367,8 @@ def rc_entries():
 
 # role files: name, header, entries, parts
 ROLE_FILES = [("rows", "rows.h", row_entries, 16), ("real_rows", "real_rows.h", real_row_entries, 16),
-              ("columns", "columns.h", column_entries, 16), ("rows_cols", "rows_cols.h", rc_entries, 8)]
+              ("columns", "columns.h", column_entries, 16), ("rows_cols", "rows_cols.h", rc_entries, 8),
+              ("planes", "planes.h", plane_entries, 8)]
 
 
 def write_roles(outdir):

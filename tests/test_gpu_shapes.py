@@ -92,3 +92,28 @@ def test_row_shapes(torch_cuda, n):
     x = oracle.uniform_complex((b, n), 0x5EED1000 + n)
     rel, _ = report(f"rows {n} x {b}", c2c(x, [n], d), oracle.c2c(x, sign_of(d)))
     assert rel <= TOL
+
+
+@pytest.mark.parametrize("n", [2, 3, 7, 8, 11, 13, 16, 20, 22, 24, 25, 26, 30, 45, 48, 50, 54, 56, 64, 81, 100, 104, 200,
+                               243, 300, 1000, 1200, 3600, 4096, 15000, 15625, 16384])
+@pytest.mark.parametrize("direction", [FWD, INV])
+def test_split_plane_rows(torch_cuda, n, direction):
+    """Rows in two planes on both sides of the line-order limit (48), one to several tiles with the last one
+    partly empty, out of place and in place."""
+    import torch
+    for b in sorted({1, max(2, min(131, (1 << 18) // n))}):
+        x = oracle.uniform_complex((b, n), 0x5EED1100 + n + b)
+        xs = [torch.from_numpy(np.ascontiguousarray(v)).cuda() for v in (x.real, x.imag)]
+        ys = [torch.empty_like(v) for v in xs]
+        h = S.FftHandle()
+        assert h.make_plan_1d(n, S.ASCEND_FFT_C2C_SEP, direction, b) == S.ACL_SUCCESS
+        h.use_current_torch_stream()
+        assert h.workspace_size() == 0
+        assert h.exec_c2c_separated(*xs, *ys) == S.ACL_SUCCESS
+        assert h.exec_c2c_separated(*xs, *xs) == S.ACL_SUCCESS
+        assert h.synchronize() == S.ACL_SUCCESS
+        h.destroy()
+        got = ys[0].cpu().numpy() + 1j * ys[1].cpu().numpy().astype(np.float64)
+        rel, _ = report(f"planes {n} x {b}", got, oracle.c2c(x, sign_of(direction)))
+        assert rel <= TOL
+        assert torch.equal(xs[0], ys[0]) and torch.equal(xs[1], ys[1])
