@@ -139,26 +139,40 @@ constexpr int last_of()
         return last_of<Rest...>();
 }
 
-// The same slice with one LDS plane (half the LDS, so that a 128 x 128 slice leaves room for a
-// second workgroup on the CU): every hand-over (HBM order -> row passes -> columns -> HBM order)
-// moves the real parts through the plane, then the imaginary parts, and the radix passes of each
-// axis are the single-plane chains of the 1D row kernel.
+// The same slice with one LDS plane (a 128 x 128 slice takes 70 KiB, so two workgroups share a CU); every exchange
+// moves the real parts through it, then the imaginary parts. The first row pass reads HBM (TY threads per
+// row, runs of TY values) and the last column pass writes HBM with lanes along y, so a slice goes through
+// three exchanges: between the row passes, rows to columns, between the column passes. Loading and
+// storing it through the plane in line order took two more: 128 x 128 x 512, 64 MiB of slices, 35.4 -> 28.9 us,
+// 128^3 x 4 60.2 -> 53.8.
 template <int X, int TX, int Y, int TY, int S, class RX, class RY>
-struct Tile2dSplit;
+struct Tile2dDirect;
 
 template <int X, int TX, int Y, int TY, int S, int... RX, int... RY>
-struct Tile2dSplit<X, TX, Y, TY, S, Radices<RX...>, Radices<RY...>> {
+struct Tile2dDirect<X, TX, Y, TY, S, Radices<RX...>, Radices<RY...>> {
     static constexpr int kThreads = (X * TY > Y * TX) ? X * TY : Y * TX;
     static constexpr int kLpy = Y + Y / 16 + 1;  // padded row pitch, [x][y] layout (odd)
     static constexpr int kLpx = X + X / 16 + 1;  // padded column pitch, [y][x] layout (odd)
     static constexpr int kPlane = (X * kLpy > Y * kLpx) ? X * kLpy : Y * kLpx;
-    static constexpr int kPer = (X * Y + kThreads - 1) / kThreads;  // elements per thread
     // first / last radix of each axis and the register shapes of those passes
     static constexpr int RY0 = first_of<RY...>(), RYL = last_of<RY...>();
     static constexpr int RX0 = first_of<RX...>(), RXL = last_of<RX...>();
     static constexpr int NBY0 = (Y / RY0 + TY - 1) / TY, NBYL = (Y / RYL + TY - 1) / TY;
-    static constexpr int NBX0 = (X / RX0 + TX - 1) / TX, NBXL = (X / RXL + TX - 1) / TX;
-    static constexpr int NSY = Y / RYL, NSX = X / RXL;  // NS of the last pass of each axis
+    static constexpr int NBX0 = (X / RX0 + TX - 1) / TX;
+    static constexpr int NSY = Y / RYL;  // NS of the last row pass
+
+    // end of the column chain: element x of column yc goes to dst[x Y]
+    struct ColOut {
+        static constexpr bool kPairTail = false;
+        static constexpr bool kRegTail = false;
+        float2 *__restrict__ out;
+        template <int R, int NS>
+        __device__ __forceinline__ void store_bf(int d, const float2 (&v)[R]) const
+        {
+#pragma unroll
+            for (int r = 0; r < R; r++) gstore(out + (d + r * NS) * Y, v[r]);
+        }
+    };
 
     __device__ __forceinline__ static void run(const StockhamArgs &a, float *pl)
     {
@@ -166,46 +180,22 @@ struct Tile2dSplit<X, TX, Y, TY, S, Radices<RX...>, Radices<RY...>> {
         const int64_t slice = blockIdx.x;
         const float2 *src = static_cast<const float2 *>(a.in) + slice * (int64_t)(X * Y);
         float2 *dst = static_cast<float2 *>(a.out) + slice * (int64_t)(X * Y);
-        // row view: transform xr (length Y), thread tr; column view: transform yc (length X), tc
+        // row view: transform xr (length Y), thread tr; column view: lanes along y, thread tc
         const int xr = tid / TY, tr = tid - xr * TY;
         const bool ract = xr < X;
-        const int yc = tid / TX, tc = tid - yc * TX;
-        const bool cact = yc < Y;
-        const int rbase = (ract ? xr : 0) * kLpy, cbase = (cact ? yc : 0) * kLpx;
+        const int tc = tid / Y, yc = tid - tc * Y;
+        const bool cact = tc < TX;
+        const int rbase = (ract ? xr : 0) * kLpy, cbase = yc * kLpx;
 
-        // HBM [x][y] -> first row pass: consecutive lanes read consecutive elements
-        const SliceMap<X, Y, kThreads> m(tid);
         float2 rin[NBY0][RY0];
-        {
-            float2 v[kPer];
 #pragma unroll
-            for (int u = 0; u < kPer; u++)
-                if (m.ok(u)) v[u] = (src + u * kThreads)[tid];
+        for (int q = 0; q < NBY0; q++) {
+            const int b = tr + q * TY;
+            if (ract && b < Y / RY0) {
 #pragma unroll
-            for (int plane = 0; plane < 2; plane++) {
-                if (plane) __syncthreads();
-#pragma unroll
-                for (int u = 0; u < kPer; u++)
-                    if (m.ok(u)) pl[m.template xy<kLpy>(u)] = plane ? v[u].y : v[u].x;
-                __syncthreads();
-#pragma unroll
-                for (int q = 0; q < NBY0; q++) {
-                    const int b = tr + q * TY;
-                    if (ract && b < Y / RY0) {
-#pragma unroll
-                        for (int r = 0; r < RY0; r++) {
-                            const float x = pl[rbase + lds_idx_read<Y / RY0>(b, r)];
-                            if (plane)
-                                rin[q][r].y = x;
-                            else
-                                rin[q][r].x = x;
-                        }
-                    }
-                }
+                for (int r = 0; r < RY0; r++) rin[q][r] = gload(src + xr * Y + b + r * (Y / RY0));
             }
-            __syncthreads();
         }
-        // row passes
         float2 rout[NBYL][RYL];
         split_chain<Y, TY, S, 1, RY...>(pl, a.tw, rbase, tr, ract, rin, RegTail<RYL>{rout});
         // row outputs (x = xr, y = j) -> [y][x] -> first column pass
@@ -243,50 +233,16 @@ struct Tile2dSplit<X, TX, Y, TY, S, Radices<RX...>, Radices<RY...>> {
             }
         }
         __syncthreads();
-        // column passes
-        float2 cout[NBXL][RXL];
-        split_chain<X, TX, S, 1, RX...>(pl, a.tw2, cbase, tc, cact, cin, RegTail<RXL>{cout});
-        // column outputs (y = yc, x = j) -> [x][y] -> HBM in order
-        float2 v[kPer];
-#pragma unroll
-        for (int plane = 0; plane < 2; plane++) {
-            __syncthreads();
-#pragma unroll
-            for (int q = 0; q < NBXL; q++) {
-                const int b = tc + q * TX;
-                if (cact && b < X / RXL) {
-                    const int k = b % NSX;
-                    const int d = (b / NSX) * NSX * RXL + k;
-#pragma unroll
-                    for (int r = 0; r < RXL; r++) {
-                        const int x = d + r * NSX;
-                        pl[x * kLpy + lds_pad(yc)] = plane ? cout[q][r].y : cout[q][r].x;
-                    }
-                }
-            }
-            __syncthreads();
-#pragma unroll
-            for (int u = 0; u < kPer; u++) {
-                if (m.ok(u)) {
-                    const float val = pl[m.template xy<kLpy>(u)];
-                    if (plane)
-                        v[u].y = val;
-                    else
-                        v[u].x = val;
-                }
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < kPer; u++)
-            if (m.ok(u)) (dst + u * kThreads)[tid] = v[u];
+        split_chain<X, TX, S, 1, RX...>(pl, a.tw2, cbase, tc, cact, cin, ColOut{dst + yc});
     }
 };
 
+// 64 registers: two 1024-thread slices per CU
 template <int X, int TX, int Y, int TY, int S, class RX, class RY>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void stockham2d_split_kernel(const StockhamArgs a)
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void stockham2d_direct_kernel(const StockhamArgs a)
 {
     extern __shared__ float lds[];
-    Tile2dSplit<X, TX, Y, TY, S, RX, RY>::run(a, lds);
+    Tile2dDirect<X, TX, Y, TY, S, RX, RY>::run(a, lds);
 }
 
 template <int X, int TX, int Y, int TY, int S, class RX, class RY>
