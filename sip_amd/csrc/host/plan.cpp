@@ -486,6 +486,8 @@ struct Builder {
             role = find_role(ROLE_ROWS, L);
         else if ((io_mode == IO_R2C_EVEN || io_mode == IO_C2R_EVEN) && flat_in && flat_out && env_flag("SIP_FFT_SPLIT_REAL", true))
             role = find_role(ROLE_REAL_ROWS, L);
+        else if ((io_mode == IO_R2C_FULL || io_mode == IO_C2R_FULL) && flat_in && flat_out && env_flag("SIP_FFT_SPLIT_REAL", true))
+            role = find_role(ROLE_REAL_ODD, L);
         // Rows in, columns out (the second four-step stage: contiguous rows of the intermediate,
         // transposed store): one plane, the first pass straight from HBM along each row, the last
         // pass straight to HBM across adjacent transforms (instead of the two-plane tile with
@@ -526,7 +528,7 @@ struct Builder {
         a.LP = lp;
         const int T = inst->T;
         const bool column = a.tin.unit_f || a.tout.unit_f;
-        const bool one_plane = role && role->role != ROLE_RC && role->role != ROLE_REAL_ROWS;
+        const bool one_plane = role != nullptr;
         const size_t per = one_plane ? (size_t)lp * 4 : (size_t)2 * lp * 4 + 24;
         int F;
         if (column) {
@@ -1271,8 +1273,10 @@ static const void *stage_kernel(const Stage &s)
     if (s.inst2d) return s.sign < 0 ? s.inst2d->fwd : s.inst2d->inv;
     if (s.rc) return s.inst->rc[s.sign < 0 ? 0 : 1];
     if (s.sa.split_lds && s.sa.col_direct) return s.inst->cols[(s.sa.tw4_ntot != 0 ? 2 : 0) + (s.sign < 0 ? 0 : 1)];
-    if (s.sa.split_lds && s.sa.io_mode == IO_R2C_EVEN) return s.inst->real_rows[s.sign < 0 ? 0 : 1];
-    if (s.sa.split_lds && s.sa.io_mode == IO_C2R_EVEN) return s.inst->real_rows[s.sign < 0 ? 2 : 3];
+    if (s.sa.split_lds && (s.sa.io_mode == IO_R2C_EVEN || s.sa.io_mode == IO_R2C_FULL))
+        return s.inst->real_rows[s.sign < 0 ? 0 : 1];
+    if (s.sa.split_lds && (s.sa.io_mode == IO_C2R_EVEN || s.sa.io_mode == IO_C2R_FULL))
+        return s.inst->real_rows[s.sign < 0 ? 2 : 3];
     if (s.planes) return s.inst->rows_fwd;
     if (s.sa.split_lds) return s.sign < 0 ? s.inst->rows_fwd : s.inst->rows_inv;
     return s.sign < 0 ? s.inst->fwd : s.inst->inv;

@@ -16,6 +16,7 @@ import sys
 
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))  # also when loaded from a path
 from column_shapes import COLUMN_SHAPES, COLUMN_TW_SHAPES, LONG_COLUMN_SHAPES
+from real_shapes import REAL_SHAPES, ROWS_COLS_SHAPES
 from row_shapes import ROW_SHAPES
 
 MAX_SMOOTH = 16384
@@ -283,18 +284,18 @@ ROWS_TWO_PLANE = {15552, 15625}
 # longest leaf used for column tiles (the host's kColumnLeafMax); every leaf up to it gets a column
 # kernel of its own (columns.h) with the shape measured for that role (column_shapes.py)
 COLUMN_LEAF_MAX = 1024
-# half lengths (with 32 or more threads per transform) of the real transforms that also get
-# single-plane R2C / C2R row kernels: every one up to 8192, and those above 8192 where the single
-# plane measured faster than the two-plane fused kernel on MI355X (R2C + C2R of 256 MiB of reals,
-# one box: 9216 155 / 211 us, 10000 161 / 226, 16384 131 / 173; it lost for most mixed lengths from
-# 12000 up, e.g. 15000 241 / 218, 13824 225 / 212)
+# half lengths of the real transforms that get single-plane R2C / C2R row kernels: from REAL_ROWS_MIN to 8192
+# with three or more threads (shorter ones are faster staged through LDS: 16 4.2 TB/s, from their own threads
+# 3.7), and those above where the single plane measured faster than the two-plane fused kernel on MI355X (R2C +
+# C2R of 256 MiB of reals, one box: 9216 155 / 211 us, 10000 161 / 226, 16384 131 / 173; it lost for most mixed
+# lengths from 12000 up, e.g. 15000 241 / 218, 13824 225 / 212)
+REAL_ROWS_MIN = 30
 REAL_ROWS_MAX = 8192
 REAL_ROWS_LONG = {8640, 9000, 9216, 9375, 9600, 9720, 10000, 10125, 10240, 10368, 10800, 10935, 11250, 11664,
                   12288, 16384}
-# lengths up to COLUMN_LEAF_MAX with two or more passes and at least this many threads per
-# transform (64-byte runs per row read) also get the rows-in / columns-out kernel of the second
-# four-step stage
-RC_MIN_THREADS = 8
+# lengths up to COLUMN_LEAF_MAX with two or more passes and at least this many threads per transform also get
+# the rows-in / columns-out kernel of the second four-step stage
+RC_MIN_THREADS = 3
 
 
 def role_entry(role, n, t, seq, f, slot, names):
@@ -338,10 +339,21 @@ def plane_entries():
 
 def real_row_entries():
     for n, t, seq in instances():
-        if n <= MAX_SMOOTH and t >= 32 and (n <= REAL_ROWS_MAX or n in REAL_ROWS_LONG):
+        t, seq, w, f = REAL_SHAPES.get(n, (t, seq, 0, 0))
+        if t >= 3 and (REAL_ROWS_MIN <= n <= REAL_ROWS_MAX or n in REAL_ROWS_LONG):
             rs = ", ".join(str(r) for r in seq)
-            yield role_entry("ROLE_REAL_ROWS", n, t, seq, 0, "real", [
-                f"stockham_real_rows_kernel<{n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)])
+            yield role_entry("ROLE_REAL_ROWS", n, t, seq, f, "real", [
+                f"stockham_real_rows_kernel<{w}, {n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)])
+
+
+# Odd lengths of the real transforms (real_odd.h), on the row kernels' shapes
+def real_odd_entries():
+    for n, t, seq in instances():
+        if n % 2 and 3 <= n <= MAX_SMOOTH:
+            t, seq = ROW_SHAPES.get(n, (t, seq))[:2]
+            rs = ", ".join(str(r) for r in seq)
+            yield role_entry("ROLE_REAL_ODD", n, t, seq, 0, "real", [
+                f"real_odd_kernel<{n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)])
 
 
 def column_entries():
@@ -360,15 +372,16 @@ def column_entries():
 
 def rc_entries():
     for n, t, seq in instances():
+        t, seq, w = ROWS_COLS_SHAPES.get(n, (t, seq, 0))
         if n <= COLUMN_LEAF_MAX and len(seq) >= 2 and t >= RC_MIN_THREADS:
             rs = ", ".join(str(r) for r in seq)
-            yield role_entry("ROLE_RC", n, t, seq, 0, "rc", [f"stockham_rc_kernel<{n}, {t}, {sg}, {rs}>" for sg in (-1, 1)])
+            yield role_entry("ROLE_RC", n, t, seq, 0, "rc", [f"stockham_rc_kernel<{w}, {n}, {t}, {sg}, {rs}>" for sg in (-1, 1)])
 
 
 # role files: name, header, entries, parts
 ROLE_FILES = [("rows", "rows.h", row_entries, 16), ("real_rows", "real_rows.h", real_row_entries, 16),
               ("columns", "columns.h", column_entries, 16), ("rows_cols", "rows_cols.h", rc_entries, 8),
-              ("planes", "planes.h", plane_entries, 8)]
+              ("planes", "planes.h", plane_entries, 8), ("real_odd", "real_odd.h", real_odd_entries, 8)]
 
 
 def write_roles(outdir):

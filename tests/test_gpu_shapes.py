@@ -9,7 +9,7 @@ import pytest
 
 import oracle
 import sip_amd as S
-from fftcase import FWD, INV, c2c, make, report, sign_of
+from fftcase import FWD, INV, c2c, c2r, make, r2c, report, sign_of
 
 pytestmark = pytest.mark.gpu
 TOL = 2e-6
@@ -117,3 +117,54 @@ def test_split_plane_rows(torch_cuda, n, direction):
         rel, _ = report(f"planes {n} x {b}", got, oracle.c2c(x, sign_of(direction)))
         assert rel <= TOL
         assert torch.equal(xs[0], ys[0]) and torch.equal(xs[1], ys[1])
+
+
+REAL = _shapes("real_shapes")
+
+
+def _real(n, b):
+    x = oracle.uniform(n * b, 0x5EED1200 + n).reshape(b, n)
+    rel, _ = report(f"r2c {n} x {b}", r2c(x, [n]), oracle.r2c(x))
+    assert rel <= TOL
+    X = oracle.uniform_complex((b, n // 2 + 1), 0x5EED1300 + n)  # imaginary parts of the end bins are dropped
+    rel, _ = report(f"c2r {n} x {b}", c2r(X, [n]), oracle.c2r(X, n))
+    assert rel <= TOL
+
+
+@pytest.mark.parametrize("L", sorted(REAL.REAL_SHAPES) + [32, 35, 64, 104, 128, 256])
+def test_real_shapes(torch_cuda, L):
+    b = max(3, min(75, (1 << 18) // L))
+    h = make([2 * L], S.ASCEND_FFT_R2C, FWD, b)
+    st = h.describe()["stages"][0]
+    h.destroy()
+    assert st["split_lds"] == 1 and (L not in REAL.REAL_SHAPES or st["T"] == REAL.REAL_SHAPES[L][0])
+    _real(2 * L, b)
+
+
+@pytest.mark.parametrize("n", [9, 15, 25, 27, 35, 45, 63, 75, 81, 99, 117, 225, 243, 375, 625, 585, 1215, 2025, 3125, 3375,
+                               3645, 6561, 9375, 10125, 15625])
+def test_real_odd_lengths(torch_cuda, n):
+    """Odd lengths, both directions of both transforms."""
+    b = max(3, min(75, (1 << 18) // n))
+    _real(n, b)
+    x = oracle.uniform(n * b, 77 + n).reshape(b, n)
+    rel, _ = report(f"r2c {n} inverse", r2c(x, [n], INV), oracle.r2c(x, oracle.INVERSE))
+    assert rel <= TOL
+    X = oracle.uniform_complex((b, n // 2 + 1), 78 + n)
+    rel, _ = report(f"c2r {n} forward", c2r(X, [n], FWD), oracle.c2r(X, n, oracle.FORWARD))
+    assert rel <= TOL
+
+
+@pytest.mark.parametrize("n", sorted(REAL.ROWS_COLS_SHAPES))
+def test_rows_cols_shapes(torch_cuda, monkeypatch, n):
+    """Second four-step stage of length n (the first factor forced)."""
+    m = next(v for v in S.smooth_lengths(33, 1024) if v * n > 32768)
+    monkeypatch.setenv("SIP_FFT_SPLIT_L1", str(m))
+    d = INV if n % 3 else FWD
+    h = make([n * m], S.ASCEND_FFT_C2C, d, 3)
+    st = h.describe()["stages"][1]
+    h.destroy()
+    assert st["L"] == n and st["rc"] == 1 and st["T"] == REAL.ROWS_COLS_SHAPES[n][0]
+    x = oracle.uniform_complex((3, n * m), 0x5EED1400 + n)
+    rel, _ = report(f"four-step {m} x {n}", c2c(x, [n * m], d), oracle.c2c(x, sign_of(d)))
+    assert rel <= TOL
