@@ -551,6 +551,14 @@ struct Builder {
             F = want > 0 ? want : pow2 ? std::min(64, std::max(16, (512 / T) & ~15)) : T >= 4 ? 16 : T >= 2 ? 32 : 64;
             if (F >= 16) F &= ~15;
             while (F > 1 && ((size_t)F * per > 160 * 1024 || F * T > 1024)) F /= 2;
+            // Few tiles: 8 wide where 16 would leave half of the CUs without one (out of place: in place, half
+            // lines written by two caches cost more than the idle CUs). Measured on MI355X, 16 / 8 wide:
+            // four-step 65536 x 1 12.2 / 9.1 us, 262144 x 4 19.3 / 16.7, 1000000 x 1 34.8 / 25.4, vertical 1024 x
+            // 512 10.8 / 8.6; at 250 tiles 100000 x 10 17.9 / 18.6; in place, 2D 1024^2 x 1 18.4 / 20.2.
+            const bool in_place = in.buf.kind == out.buf.kind && in.buf.ws_index == out.buf.ws_index;
+            // Gathered groups keep 16: other launches run beside them.
+            if (want <= 0 && !mf && !in_place && a.tin.tab_dim < 0 && a.tout.tab_dim < 0 && (nfft + 15) / 16 <= 128)
+                F = std::min(F, 8);
         } else {
             F = role && role->F ? role->F : std::max(1, 256 / T);
             while (F > 1 && ((size_t)F * per > 48 * 1024 || F * T > 1024)) F--;
