@@ -13,6 +13,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../kernels/aux_args.h"
@@ -190,6 +191,8 @@ std::string plan_describe(const Plan &p);
 const StockhamInstance *find_instance(int64_t L);
 // Single-plane kernels of a role and length, or null.
 const RoleInstance *find_role(Role role, int64_t L);
+// Measured GB/s of a length as first and second four-step stage (0, 0: not measured).
+std::pair<int, int> split_rates(int64_t L);
 // Split-precision MFMA instances (mode = PrecisionMode) and their DFT-matrix operand table.
 const StockhamInstance *find_mfma_instance(int64_t L, int mode);
 // Fused 2D tile instance for X x Y slices (X, Y in 32, 64, 128), or null.

@@ -80,6 +80,15 @@ const RoleInstance *find_role(Role role, int64_t L)
     return it == m.end() ? nullptr : it->second;
 }
 
+std::pair<int, int> split_rates(int64_t L)
+{
+    static const std::map<int64_t, std::pair<int, int>> m = {
+#include "split_rates.inc"
+    };
+    auto it = m.find(L);
+    return it == m.end() ? std::pair<int, int>{0, 0} : it->second;
+}
+
 #define SIP_ISTFT_PART(k)                            \
     extern const IstftInstance g_istft_part_##k[];   \
     extern const int g_istft_part_##k##_count;

@@ -18,6 +18,7 @@ sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))  # also when load
 from column_shapes import COLUMN_SHAPES, COLUMN_TW_SHAPES, LONG_COLUMN_SHAPES
 from real_shapes import REAL_SHAPES, ROWS_COLS_SHAPES
 from row_shapes import ROW_SHAPES
+from split_rates import SPLIT_RATES
 
 MAX_SMOOTH = 16384
 MAX_POW2 = 16384
@@ -396,6 +397,9 @@ def write_roles(outdir):
             write_if_changed(os.path.join(outdir, f"{name}_part_{k}.hip"), "\n".join(text) + "\n")
             inc.append(f"SIP_ROLE_PART({name}_part_{k})")
     write_if_changed(os.path.join(outdir, "role_parts.inc"), "\n".join(inc) + "\n")
+    rates = ["// Generated by gen_instances.py (do not edit): length, first and second four-step stage in GB/s."]
+    rates += [f"{{{n}, {{{a}, {b}}}}}," for n, (a, b) in sorted(SPLIT_RATES.items())]
+    write_if_changed(os.path.join(outdir, "split_rates.inc"), "\n".join(rates) + "\n")
 
 
 # One-launch inverse short-time transforms (istft.h): every 2,3,5-smooth frame length in this range,

@@ -168,3 +168,16 @@ def test_rows_cols_shapes(torch_cuda, monkeypatch, n):
     x = oracle.uniform_complex((3, n * m), 0x5EED1400 + n)
     rel, _ = report(f"four-step {m} x {n}", c2c(x, [n * m], d), oracle.c2c(x, sign_of(d)))
     assert rel <= TOL
+
+
+@pytest.mark.parametrize("n, factors", [(243000, [675, 360]), (327680, [640, 512]), (777600, [960, 810]),
+                                        (65536, [256, 256])])
+def test_four_step_splits_by_measured_rates(torch_cuda, n, factors):
+    """Splits that the stage rates choose (split_rates.py) and one that they leave alone."""
+    for d in (FWD, INV):
+        h = make([n], S.ASCEND_FFT_C2C, d, 2)
+        assert [s["L"] for s in h.describe()["stages"]] == factors
+        h.destroy()
+        x = oracle.uniform_complex((2, n), 0x5EED1100 + n)
+        rel, _ = report(f"split {n}", c2c(x, [n], d), oracle.c2c(x, sign_of(d)))
+        assert rel <= TOL
