@@ -10,12 +10,14 @@
 //     transposes, fft_api.cpp:478-483, 527-697);
 //   * a longer axis runs as a four-step pair L = L1 * L2 (column FFTs with the W_L^{l2 k1}
 //     twiddle folded into their store, then row FFTs that store transposed), recursively;
-//   * a length with a prime factor above 13 runs through Bluestein's chirp-z convolution with
-//     power-of-two FFTs (the reference's generic matrix core FFTCoreAny, fft_core_any.cpp:282-589,
-//     plays that role there);
+//   * a length with a prime factor above 13 runs through Bluestein's chirp-z convolution (the
+//     reference's generic matrix core FFTCoreAny, fft_core_any.cpp:282-589, plays that role there):
+//     stages with power-of-two FFTs, one launch on 2,3,5-smooth FFTs up to 16384 points;
 //   * even-length real transforms run a half-length complex FFT with the split post- / pre-process
 //     fused into the same launch when the half length is a leaf (reference A/B tables,
 //     core/fft/fftcore/fft_core_common_func.cpp:569-673).
+// Where one launch stands for a run of stages (Plan::fusions), the stages remain what the plan
+// describes and what its workspace is sized for.
 #include "plan.h"
 
 #include <algorithm>
@@ -435,36 +437,36 @@ struct Builder {
                env_flag("SIP_FFT_BIG_LEAF", true);
     }
 
-    // Columns of 1025 to 4096 points in one pass of the long column kernels instead of the two four-step
-    // passes, from 128 tiles up (half of the CUs). Measured on MI355X, two passes / one, 64 MiB of columns:
-    // 1080 60 / 35 us, 2048 56 / 30, 4096 54 / 42; fewer tiles leave the chip to a few long workgroups: 2048
-    // x 100 columns (7 tiles) 9 / 19 us, R2C 1080 x 1920 (61 tiles) 26 / 28 us, C2C 2048 x 2048 (128) 44 / 37.
     // Contiguous transforms of length L, each starting where the one before ends
     static bool whole_rows(const TileDesc &t, int64_t L)
     {
         return t.es == 1 && t.tab_dim < 0 && t.n1 == 1 && (t.n0 == 1 || t.s0 == L);
     }
 
+    // Columns of 1025 to 4096 points in one pass of the long column kernels instead of the two four-step
+    // passes, from 128 tiles up (half of the CUs). Measured on MI355X, two passes / one, 64 MiB of columns:
+    // 1080 60 / 35 us, 2048 56 / 30, 4096 54 / 42; fewer tiles leave the chip to a few long workgroups: 2048
+    // x 100 columns (7 tiles) 9 / 19 us, R2C 1080 x 1920 (61 tiles) 26 / 28 us, C2C 2048 x 2048 (128) 44 / 37.
     bool long_columns(int64_t L, const Lay &in, const Lay &out) const
     {
         const RoleInstance *ci = L > kColumnLeafMax ? find_role(ROLE_COLS, L) : nullptr;
         bool ok = true;
         int tab;
-        return ci && p.precision == PREC_FP32 && !is_user(in.buf) && !is_user(out.buf) &&
+        return ci && !is_user(in.buf) && !is_user(out.buf) &&
                to_tile(in, &ok, &tab).unit_f && to_tile(out, &ok, &tab).unit_f && ok &&
                count(normalize(in.dims)) >= 128 * (int64_t)ci->F && split_columns(L) &&
                env_flag("SIP_FFT_COL_DIRECT", true);
     }
 
     void add_stockham(int64_t L, int sign, const Lay &in, const Lay &out, int io_mode, int64_t in_len,
-                      int64_t out_len, int64_t tw4_ntot, int64_t col_div, const std::string &note)
+                      int64_t out_len, int64_t tw4_ntot, int64_t col_div, const std::string &note, bool fp32 = false)
     {
         const StockhamInstance *inst = find_instance(L);
         // precision form: C2C launches with radix-16 stages run them on the matrix cores
         const bool in_sep = is_user(in.buf), out_sep = is_user(out.buf);
         if ((in_sep || out_sep) && io_mode != IO_C2C)
             throw SipError(AsdSip::ACL_ERROR_INTERNAL_ERROR, "split planes on a real-transform stage");
-        const StockhamInstance *mf = (p.precision != PREC_FP32 && io_mode == IO_C2C && !in_sep && !out_sep)
+        const StockhamInstance *mf = (p.precision != PREC_FP32 && !fp32 && io_mode == IO_C2C && !in_sep && !out_sep)
                                          ? find_mfma_instance(L, p.precision) : nullptr;
         if (mf) inst = mf;
         bool ok = true;
@@ -888,9 +890,14 @@ struct Builder {
         Lay bin{mid.buf, mid.es, with_dim(mid.dims, posB, {L1, mid.es * L2})};
         Lay bout{out.buf, out.es * L1, with_dim(out.dims, posB, {L1, out.es})};
         axis(L2, sign, bin, bout, true, depth + 1);
-        if (depth == 0 && forced <= 1 && fusing() && long_columns(L, in, out)) {
+        // In the precision form too, where no stage of the split runs on the matrix cores: one FP32 launch for two.
+        // 2D on MI355X, two launches / one: f16 hi + lo 2048 x 2048 x 2 86.7 / 64.8 us, 2048 x 512 x 8 79.0 / 62.9,
+        // 1536 x 1024 x 4 63.1 / 50.0; bf16 hi + mid + lo 2048 x 2048 x 2 85.6 / 64.7.
+        const bool fp32_split = std::none_of(p.stages.begin() + first, p.stages.end(),
+                                             [](const Stage &s) { return s.mfw.used(); });
+        if (depth == 0 && forced <= 1 && fusing() && fp32_split && long_columns(L, in, out)) {
             const size_t last = p.stages.size() - 1;
-            add_stockham(L, sign, in, out, IO_C2C, L, L, 0, 1, "columns " + std::to_string(L));
+            add_stockham(L, sign, in, out, IO_C2C, L, L, 0, 1, "columns " + std::to_string(L), true);
             Stage st = std::move(p.stages.back());
             p.stages.pop_back();
             p.fusions.push_back(Fusion{first, last, std::move(st)});

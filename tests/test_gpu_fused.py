@@ -8,7 +8,7 @@ import pytest
 
 import oracle
 import sip_amd as S
-from fftcase import FWD, INV, report, sign_of
+from fftcase import FWD, INV, c2c, make, report, sign_of
 
 pytestmark = pytest.mark.gpu
 AGREE = 1e-6
@@ -126,3 +126,18 @@ def test_istft_one_launch(torch_cuda, monkeypatch, ch, n, hop, frames):
 
     got, staged = _both(lambda h: h.istft_make_plan(xd, n, hop, n), execute, monkeypatch)
     _agree(f"istft ch={ch} n={n} hop={hop} frames={frames}", got, staged, oracle.istft(x, n, hop, w), 2e-6)
+
+@pytest.mark.parametrize("mode", [S.PREC_F16_SPLIT, S.PREC_BF16_SPLIT3])
+@pytest.mark.parametrize("a, b, batch", [(2048, 525, 4), (1536, 1050, 2)])
+def test_precision_long_columns(torch_cuda, monkeypatch, a, b, batch, mode):
+    """An axis whose four-step stages are FP32 in the precision form too runs as one FP32 column pass there
+    (counts that leave the last tile partly empty); both agree with the oracle as FP32 does."""
+    x = oracle.uniform_complex((batch, a, b), 0x5EED1500 + a)
+    want = oracle.c2c_nd(x, 2, sign_of(INV))
+    for fuse in ("1", "0"):
+        monkeypatch.setenv("SIP_FFT_FUSE", fuse)
+        h = make([a, b], S.ASCEND_FFT_C2C, INV, batch, precision=mode)
+        assert len(h.describe()["fused"]) == int(fuse)
+        h.destroy()
+        rel, _ = report(f"{a} x {b} fuse={fuse}", c2c(x, [a, b], INV, precision=mode), want)
+        assert rel <= 2e-6
