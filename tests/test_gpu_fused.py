@@ -107,10 +107,13 @@ def test_bluestein_split_planes(torch_cuda, monkeypatch, n, b):
 
 
 # one frame more than a tile holds, fewer frames than the halo, hops that divide the frame and that do
-# not, no overlap at all, odd lengths, the shortest hop that is still one launch (n / 8 with 16 frames)
+# not, no overlap at all, odd lengths, the shortest hop that is still one launch (n / 8 with 16 frames), tiles
+# of few frames
 @pytest.mark.parametrize("ch,n,hop,frames", [(1, 24, 6, 65), (2, 27, 10, 40), (3, 256, 64, 2), (2, 256, 256, 70),
                                              (2, 400, 160, 131), (1, 625, 125, 9), (2, 1024, 256, 17),
-                                             (1, 1024, 128, 33), (2, 1080, 270, 20), (1, 1458, 365, 12)])
+                                             (1, 1024, 128, 33), (2, 1080, 270, 20), (1, 1458, 365, 12),
+                                             (1, 1440, 720, 164), (1, 1440, 360, 165), (4, 640, 320, 103),
+                                             (16, 1200, 600, 90), (1, 960, 960, 31)])
 def test_istft_one_launch(torch_cuda, monkeypatch, ch, n, hop, frames):
     import torch
     rng = np.random.default_rng(n * 7 + hop)
@@ -126,6 +129,7 @@ def test_istft_one_launch(torch_cuda, monkeypatch, ch, n, hop, frames):
 
     got, staged = _both(lambda h: h.istft_make_plan(xd, n, hop, n), execute, monkeypatch)
     _agree(f"istft ch={ch} n={n} hop={hop} frames={frames}", got, staged, oracle.istft(x, n, hop, w), 2e-6)
+
 
 @pytest.mark.parametrize("mode", [S.PREC_F16_SPLIT, S.PREC_BF16_SPLIT3])
 @pytest.mark.parametrize("a, b, batch", [(2048, 525, 4), (1536, 1050, 2)])
