@@ -558,8 +558,10 @@ struct Builder {
             // four-step 65536 x 1 12.2 / 9.1 us, 262144 x 4 19.3 / 16.7, 1000000 x 1 34.8 / 25.4, vertical 1024 x
             // 512 10.8 / 8.6; at 250 tiles 100000 x 10 17.9 / 18.6; in place, 2D 1024^2 x 1 18.4 / 20.2.
             const bool in_place = in.buf.kind == out.buf.kind && in.buf.ws_index == out.buf.ws_index;
-            // Gathered groups keep 16: other launches run beside them.
-            if (want <= 0 && !mf && !in_place && a.tin.tab_dim < 0 && a.tout.tab_dim < 0 && (nfft + 15) / 16 <= 128)
+            // Gathered groups keep 16: other launches run beside them. A tile still fills a wave: below 8 threads per
+            // transform the 8-wide one leaves lanes idle and reads half lines for nothing (vertical 80 x 512 as 4 threads
+            // 4.6 / 5.3 us, 36 x 1000 3.5 / 4.0, 16 x 1000 2.6 / 2.9).
+            if (want <= 0 && !mf && !in_place && 8 * T >= 64 && a.tin.tab_dim < 0 && a.tout.tab_dim < 0 && (nfft + 15) / 16 <= 128)
                 F = std::min(F, 8);
         } else {
             F = role && role->F ? role->F : std::max(1, 256 / T);
@@ -637,8 +639,10 @@ struct Builder {
         // lines, which two L2s would fetch and write apart: XCD-contiguous tile order. Measured on
         // MI355X, launch / XCD-contiguous order, columns of 64 MiB: 100 x 83886 35.2 / 26.7 us, 243 x
         // 34521 38.9 / 28.1, 1080 x 7767 42.4 / 36.8, R2C 512^2 x 64 68.9 / 54.9; whole lines lose by it:
-        // 256 x 32768 22.8 / 25.0, 1024 x 8192 25.8 / 27.9; so do rows (4096 x 16384 0.194 / 0.200 ms).
-        const bool split_lines = (a.tin.unit_f && a.tin.es % 16 != 0) || (a.tout.unit_f && a.tout.es % 16 != 0);
+        // 256 x 32768 22.8 / 25.0, 1024 x 8192 25.8 / 27.9; so do rows (4096 x 16384 0.194 / 0.200 ms). Column tiles 8
+        // wide share every line: 512 x 2048 9.15 / 7.73 us, 360 x 2048 8.85 / 7.27, 1500 x 4096 29.8 / 27.3, 1920 x 4096
+        // 48.9 / 44.0; 8-wide tiles of rows lose (four-step 262144 x 8 21.8 / 25.6, 1048576 x 2 25.5 / 29.4).
+        const bool split_lines = (a.tin.unit_f && (a.tin.es % 16 != 0 || F % 16 != 0)) || (a.tout.unit_f && a.tout.es % 16 != 0);
         a.xcd_remap = p.tune.xcd >= 0 ? p.tune.xcd == 1 : env_flag("SIP_FFT_XCD", column && split_lines);
         // matrix passes read [k][16] twiddle rows; the single-plane rows kernel (K = 32) reads the
         // interleaved operand table, the two-plane tile (K = 16) the blocked one
