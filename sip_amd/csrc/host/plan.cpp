@@ -375,6 +375,7 @@ static int64_t big_leaf_min_rows(const Plan &p)
 // One launch for a run of stages where a fused kernel exists; SIP_FFT_FUSE=0 at plan time runs the
 // stages one by one (the comparison path of the tests).
 static bool fusing() { return env_flag("SIP_FFT_FUSE", true); }
+static bool fusing_always() { return env_flag("SIP_FFT_FUSE", false); }
 
 // LDS pitch (floats) of a transform of n values padded by one word every 16, odd.
 static int lds_pitch(int64_t n)
@@ -931,7 +932,10 @@ struct Builder {
     void fuse(size_t first, Stage &&st) { p.fusions.push_back(Fusion{first, p.stages.size() - 1, std::move(st)}); }
 
     // One-launch Bluestein (kernels/bluestein.h) for every length whose convolution fits an
-    // instance (N <= 16384), any strides; the precision form keeps its matrix-core FFT stages.
+    // instance (N <= 16384), any strides; the precision form keeps its matrix-core FFT stages. The longest
+    // convolutions stay stages for few transforms (BluesteinInstance::rows, cols), except where the arithmetic must
+    // not depend on their number (p.big_leaf), in gathered groups, beside which other launches run, and with
+    // SIP_FFT_FUSE=1.
     void fuse_bluestein(size_t first, int64_t N, int sign, const Lay &in, const Lay &out)
     {
         const BluesteinInstance *bi = p.precision == PREC_FP32 ? find_bluestein_instance(2 * N - 1) : nullptr;
@@ -949,6 +953,9 @@ struct Builder {
         a.tout = to_tile(out, &ok, &st.out_tab);
         a.nfft = count(normalize(in.dims));
         if (!ok || a.nfft >= (int64_t(1) << 31)) return;
+        a.col_direct = (a.tin.unit_f || a.tout.unit_f) ? 1 : 0;
+        const int64_t from = a.col_direct ? bi->cols : bi->rows;
+        if (a.nfft < from && p.big_leaf && a.tin.tab_dim < 0 && !fusing_always()) return;
         a.tin.vec2 = a.tout.vec2 = 0;
         a.io_mode = IO_C2C;
         a.in_len = a.out_len = (int32_t)N;
@@ -957,16 +964,18 @@ struct Builder {
         a.LP = lds_pitch(bi->M);
         const int T = bi->T;
         const int64_t per = (int64_t)a.LP * 4;
-        // Column tiles (lanes walk adjacent transforms) 16 wide, rows about 256 threads; fewer rows per
-        // workgroup until the grid has two workgroups per CU, as for the leaf kernels.
-        a.col_direct = (a.tin.unit_f || a.tout.unit_f) ? 1 : 0;
+        // Column tiles (lanes walk adjacent transforms) 16 wide, rows about 256 threads; fewer transforms per
+        // workgroup until the grid has two workgroups per CU, as for the leaf kernels. Columns too: a transform's
+        // chain of passes outlasts what its narrow reads cost (1009 x 32 columns 16 / 1 wide 24.3 / 8.4 us, 2039 x 256
+        // 4 / 1 wide 28 / 13, 1009 x 1024 16 / 2 wide 26 / 16; in launch order 8191 x 64 44, in XCD order 35).
         int F = a.col_direct ? 16 : std::max(1, 256 / T);
         while (F > 1 && (F * T > 1024 || F * per > (a.col_direct ? 160 : 48) * 1024)) F = (F + 1) / 2;
-        if (!a.col_direct)
-            while (F > 1 && ((F + 1) / 2) * T >= 64 && (a.nfft + F - 1) / F < kFillWorkgroups) F = (F + 1) / 2;
+        while (F > 1 && ((F + 1) / 2) * T >= 64 && (a.nfft + F - 1) / F < kFillWorkgroups) F = (F + 1) / 2;
         if (F > a.nfft) F = (int)a.nfft;
         a.F = F;
         a.div_F = make_fastdiv((uint32_t)F);
+        // adjacent column tiles share lines unless they are whole ones: XCD-contiguous order (as add_stockham)
+        a.xcd_remap = a.col_direct && (F % 16 != 0 || (a.tin.unit_f && a.tin.es % 16 != 0));
         std::vector<int> rad(bi->radix, bi->radix + bi->npass);
         st.tw = pass_twiddles_seq(bi->M, rad, -1);
         std::reverse(rad.begin(), rad.end());

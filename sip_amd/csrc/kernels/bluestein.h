@@ -81,7 +81,7 @@ struct Bluestein<M, T, Radices<RF...>, Radices<RI...>> {
             flp = tid / T;
             t = tid - flp * T;
         }
-        const int64_t f = (int64_t)blockIdx.x * F + flp;
+        const int64_t f = tile_index(a) * F + flp;
         const bool active = f < a.nfft;
         int64_t ib = 0, ob = 0;  // a lane without a transform reads transform 0's elements, stores none
         if (active) {

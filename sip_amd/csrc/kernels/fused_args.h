@@ -12,6 +12,7 @@ struct BluesteinInstance {
     int32_t M, T, npass;
     int32_t radix[4];
     const void *fn;
+    int32_t rows, cols;  // rows / adjacent columns from which the one launch is faster than the stages
 };
 
 // Contiguous R2C / C2R rows of odd length (real_odd.h); real_rows[] as for ROLE_REAL_ROWS.

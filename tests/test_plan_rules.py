@@ -22,3 +22,22 @@ def test_column_tiles_of_few_columns(n, b):
         assert st["T"] >= 8 and st["xcd_remap"] == 1
     else:
         assert st["F"] >= 16 and st["T"] < 8
+
+
+@pytest.mark.parametrize("n,rows,cols", [(31, 1, 1), (1009, 1, 1), (8191, 1, 1), (9973, 12, 24), (12277, 16, 48), (16381, 24, 64)])
+def test_bluestein_of_few_transforms(n, rows, cols, monkeypatch):
+    """The longest convolutions stay stages below the measured number of transforms; SIP_FFT_FUSE=1 runs them
+    in one launch all the same."""
+    monkeypatch.delenv("SIP_FFT_FUSE", raising=False)
+    for b, dim in ((rows, S.ASCEND_FFT_HORIZONTAL), (cols, VERT)):
+        assert len(S.describe_dry([n], C2C, FWD, b, dim)["fused"]) == 1
+        if b > 1:
+            assert S.describe_dry([n], C2C, FWD, b - 1, dim)["fused"] == []
+    monkeypatch.setenv("SIP_FFT_FUSE", "1")
+    assert len(columns(n, 2)["fused"]) == 1
+
+
+@pytest.mark.parametrize("n,b,grid", [(251, 32, 32), (509, 256, 256), (1009, 32, 32), (2039, 4, 4), (1009, 4096, 512)])
+def test_bluestein_columns_fill_the_chip(n, b, grid):
+    """Column tiles narrow until the launch has two workgroups per CU, down to one transform each."""
+    assert columns(n, b)["fused"][0]["grid"] >= grid
