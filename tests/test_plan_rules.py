@@ -41,3 +41,16 @@ def test_bluestein_of_few_transforms(n, rows, cols, monkeypatch):
 def test_bluestein_columns_fill_the_chip(n, b, grid):
     """Column tiles narrow until the launch has two workgroups per CU, down to one transform each."""
     assert columns(n, b)["fused"][0]["grid"] >= grid
+
+
+@pytest.mark.parametrize("n,width", [(3, 64), (20, 64), (24, 32), (40, 32), (36, 16), (45, 16), (60, 16), (81, 16), (1000, 16)])
+def test_column_tile_widths(n, width):
+    """Many columns: whole waves for one or two threads per column, whole lines otherwise."""
+    assert columns(n, 8192)["stages"][0]["F"] == width
+
+
+def test_split_stages_cut_columns_alike():
+    """A split axis of few-thread factors keeps one tile width in both launches."""
+    for n in (1080, 1200):
+        st = S.describe_dry([n, 1024], C2C, FWD, 1)["stages"][1:]
+        assert len(st) == 2 and [s["F"] for s in st] == [16, 16]
