@@ -322,8 +322,13 @@ def row_entries():
         yield role_entry("ROLE_ROWS", n, t, seq, f, "rows", [f"stockham_rows_kernel<{w}, {n}, {t}, {sg}, {rs}>" for sg in (-1, 1)])
 
 
-# Split-plane rows up to this length go through LDS in line order (planes.h)
+# Split-plane rows up to this length go through LDS in line order (planes.h), on the leaf's threads but for these:
+# 40 and 45 points on two and three threads spilled (116 and 48 bytes a lane; 40 x 4096 16.0 us, on eight threads
+# 3.7), 33 and 39 took 97 and 115 registers (33 x 64 7.0 / 3.8). 65 and 66 points, also in line order, ran 64 MiB from
+# their own five and six threads in 57.7 and 52.0 us.
 PLANES_SMALL_MAX = 48
+PLANES_SMALL_SHAPES = {33: (11, [11, 3]), 39: (13, [13, 3]), 40: (8, [8, 5]), 45: (9, [9, 5]), 52: (13, [13, 4]),
+                       65: (13, [13, 5]), 66: (11, [11, 6])}
 
 
 def plane_entries():
@@ -331,10 +336,13 @@ def plane_entries():
         if n > MAX_SMOOTH:
             continue
         w, f = 0, 0
-        if n > PLANES_SMALL_MAX:
+        small = n <= PLANES_SMALL_MAX or n in PLANES_SMALL_SHAPES
+        if small:
+            t, seq = PLANES_SMALL_SHAPES.get(n, (t, seq))
+        else:
             t, seq, w, f = ROW_SHAPES.get(n, (t, seq, 0, 0))
         rs = ", ".join(str(r) for r in seq)
-        name = f"planes_small_kernel<{n}, {t}, {rs}>" if n <= PLANES_SMALL_MAX else f"planes_rows_kernel<{w}, {n}, {t}, {rs}>"
+        name = f"planes_small_kernel<{n}, {t}, {rs}>" if small else f"planes_rows_kernel<{w}, {n}, {t}, {rs}>"
         yield role_entry("ROLE_PLANES", n, t, seq, f, "rows", [name, "nullptr"])
 
 

@@ -94,7 +94,8 @@ def test_row_shapes(torch_cuda, n):
     assert rel <= TOL
 
 
-@pytest.mark.parametrize("n", [2, 3, 7, 8, 11, 13, 16, 20, 22, 24, 25, 26, 30, 45, 48, 50, 54, 56, 64, 81, 100, 104, 200,
+@pytest.mark.parametrize("n", [2, 3, 7, 8, 11, 13, 16, 20, 22, 24, 25, 26, 30, 33, 39, 40, 45, 48, 50, 52, 54, 56, 64, 65, 66, 81,
+                               100, 104, 200,
                                243, 300, 1000, 1200, 3600, 4096, 15000, 15625, 16384])
 @pytest.mark.parametrize("direction", [FWD, INV])
 def test_split_plane_rows(torch_cuda, n, direction):
