@@ -445,9 +445,10 @@ struct Builder {
     }
 
     // Columns of 1025 to 4096 points in one pass of the long column kernels instead of the two four-step
-    // passes, from 128 tiles up (half of the CUs). Measured on MI355X, two passes / one, 64 MiB of columns:
-    // 1080 60 / 35 us, 2048 56 / 30, 4096 54 / 42; fewer tiles leave the chip to a few long workgroups: 2048
-    // x 100 columns (7 tiles) 9 / 19 us, R2C 1080 x 1920 (61 tiles) 26 / 28 us, C2C 2048 x 2048 (128) 44 / 37.
+    // passes, from 128 tiles up (half of the CUs; some lengths later, column_shapes.py). Measured on MI355X, two
+    // passes / one: 1080 x 2048 columns 21.8 / 15.9 us, 1500 x 2048 23.6 / 16.6, 2048 x 2048 29.1 / 22.4, 64 MiB of
+    // 1080 60 / 35, of 2048 56 / 30; fewer tiles leave the chip to a few long workgroups: 2048 x 100 columns (7 tiles)
+    // 9 / 19 us, R2C 1080 x 1920 (61 tiles) 26 / 28 us.
     bool long_columns(int64_t L, const Lay &in, const Lay &out) const
     {
         const RoleInstance *ci = L > kColumnLeafMax ? find_role(ROLE_COLS, L) : nullptr;
@@ -455,7 +456,7 @@ struct Builder {
         int tab;
         return ci && !is_user(in.buf) && !is_user(out.buf) &&
                to_tile(in, &ok, &tab).unit_f && to_tile(out, &ok, &tab).unit_f && ok &&
-               count(normalize(in.dims)) >= 128 * (int64_t)ci->F && split_columns(L) &&
+               count(normalize(in.dims)) >= ci->from * (int64_t)ci->F && split_columns(L) &&
                env_flag("SIP_FFT_COL_DIRECT", true);
     }
 
@@ -481,23 +482,35 @@ struct Builder {
         // Contiguous rows of plain C2C stages: the row kernels' own threads and radices (every first and last
         // pass straight from / to HBM), unless the tuner or SIP_FFT_SPLIT_LDS=0 asks for the two-plane leaf.
         const bool flat_in = tin.es == 1 && !tin.unit_f && !in_sep, flat_out = tout.es == 1 && !tout.unit_f && !out_sep;
+        const int64_t nfft = count(normalize(in.dims));
+        // A shape that needs many workgroups: gathered groups have other launches beside them, and where the
+        // arithmetic must not depend on the number of transforms (!p.big_leaf) the leaf is for all.
+        auto enough = [&](const RoleInstance *r, int64_t width) {
+            if (!r || r->from == 0) return true;
+            return p.big_leaf && (tin.tab_dim >= 0 || nfft >= (r->from - 1) * width + 1);
+        };
         const RoleInstance *role = nullptr;
-        if (columns && !mf && split_columns(L))
+        if (columns && !mf && split_columns(L)) {
             role = find_role(tw4_ntot != 0 ? ROLE_COLS_TW : ROLE_COLS, L);
-        else if (io_mode == IO_C2C && !mf && flat_in && flat_out && tw4_ntot == 0 && (L > kRowLeafMax || p.tune.split_lds != 0) &&
-                 (L > kRowLeafMax || env_flag("SIP_FFT_SPLIT_LDS", true)))
+            if (L <= kColumnLeafMax && !enough(role, 16)) role = nullptr;
+        } else if (io_mode == IO_C2C && !mf && flat_in && flat_out && tw4_ntot == 0 && (L > kRowLeafMax || p.tune.split_lds != 0) &&
+                 (L > kRowLeafMax || env_flag("SIP_FFT_SPLIT_LDS", true))) {
             role = find_role(ROLE_ROWS, L);
-        else if ((io_mode == IO_R2C_EVEN || io_mode == IO_C2R_EVEN) && flat_in && flat_out && env_flag("SIP_FFT_SPLIT_REAL", true))
+            if (p.tune.split_lds != 1 && !enough(role, 1)) role = nullptr;
+        } else if ((io_mode == IO_R2C_EVEN || io_mode == IO_C2R_EVEN) && flat_in && flat_out && env_flag("SIP_FFT_SPLIT_REAL", true)) {
             role = find_role(ROLE_REAL_ROWS, L);
-        else if ((io_mode == IO_R2C_FULL || io_mode == IO_C2R_FULL) && flat_in && flat_out && env_flag("SIP_FFT_SPLIT_REAL", true))
+            if (!enough(role, 1)) role = nullptr;
+        } else if ((io_mode == IO_R2C_FULL || io_mode == IO_C2R_FULL) && flat_in && flat_out && env_flag("SIP_FFT_SPLIT_REAL", true))
             role = find_role(ROLE_REAL_ODD, L);
         // Rows in, columns out (the second four-step stage: contiguous rows of the intermediate,
         // transposed store): one plane, the first pass straight from HBM along each row, the last
         // pass straight to HBM across adjacent transforms (instead of the two-plane tile with
         // LDS-staged store).
         else if (io_mode == IO_C2C && !mf && flat_in && tout.unit_f && !out_sep && tw4_ntot == 0 &&
-                 (p.tune.rc >= 0 ? p.tune.rc == 1 : env_flag("SIP_FFT_RC", true)))
+                 (p.tune.rc >= 0 ? p.tune.rc == 1 : env_flag("SIP_FFT_RC", true))) {
             role = find_role(ROLE_RC, L);
+            if (p.tune.rc != 1 && !enough(role, 16)) role = nullptr;
+        }
         // Split planes on both sides, rows one after the other (the kernel of up to 48 points reads them as one run)
         else if (io_mode == IO_C2C && in_sep && out_sep && tw4_ntot == 0 && whole_rows(tin, L) && whole_rows(tout, L) &&
                  env_flag("SIP_FFT_SPLIT_LDS", true))
@@ -516,7 +529,6 @@ struct Builder {
         a.tin = tin;
         a.tout = tout;
         if (!ok) throw SipError(AsdSip::ACL_ERROR_API_NOT_SUPPORT, "layout has more than 3 batch dimensions");
-        const int64_t nfft = count(normalize(in.dims));
         if (nfft != count(normalize(out.dims)))
             throw SipError(AsdSip::ACL_ERROR_INTERNAL_ERROR, "stage in/out transform counts differ");
         if (nfft >= (int64_t(1) << 31))

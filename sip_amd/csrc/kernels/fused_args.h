@@ -15,9 +15,6 @@ struct BluesteinInstance {
     int32_t rows, cols;  // rows / adjacent columns from which the one launch is faster than the stages
 };
 
-// Contiguous R2C / C2R rows of odd length (real_odd.h); real_rows[] as for ROLE_REAL_ROWS.
-constexpr Role ROLE_REAL_ODD = static_cast<Role>(6);
-
 // One-launch inverse short-time transform (istft.h).
 struct IstftArgs {
     const float2 *in;     // spectra (channel, n, frames)

@@ -15,9 +15,9 @@ import os
 import sys
 
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))  # also when loaded from a path
-from column_shapes import COLUMN_SHAPES, COLUMN_TW_SHAPES, LONG_COLUMN_SHAPES
-from real_shapes import REAL_SHAPES, ROWS_COLS_SHAPES
-from row_shapes import ROW_SHAPES
+from column_shapes import COLUMN_FROM, COLUMN_SHAPES, COLUMN_TW_FROM, COLUMN_TW_SHAPES, LONG_COLUMN_FROM, LONG_COLUMN_SHAPES
+from real_shapes import REAL_SHAPES, ROWS_COLS_FROM, ROWS_COLS_SHAPES
+from row_shapes import ROW_FROM, ROW_SHAPES
 from split_rates import SPLIT_RATES
 
 MAX_SMOOTH = 16384
@@ -277,10 +277,10 @@ def instances():
 
 # Contiguous-row kernels (rows.h) from ROWS_MIN points up, with three or more threads per transform: shorter
 # rows, and leaves of fewer threads, are faster staged through LDS in line order (16: 5.3-6.0 TB/s staged,
-# 4.1 from their own threads). Two lengths are faster on the two-plane tile: 256 MiB of rows, single / two
-# planes, 15625 268 / 240 us, 15552 171 / 158.
+# 4.1 from their own threads). Three lengths are faster on the two-plane tile: 256 MiB of rows, single / two
+# planes, 15625 268 / 240 us, 15552 171 / 158; 8748 (512 rows 21.7 / 20.5, 700 rows 30.7 / 31.3).
 ROWS_MIN, ROWS_MIN_THREADS = 24, 3
-ROWS_TWO_PLANE = {15552, 15625}
+ROWS_TWO_PLANE = {8748, 15552, 15625}
 
 # longest leaf used for column tiles (the host's kColumnLeafMax); every leaf up to it gets a column
 # kernel of its own (columns.h) with the shape measured for that role (column_shapes.py)
@@ -299,8 +299,8 @@ REAL_ROWS_LONG = {8640, 9000, 9216, 9375, 9600, 9720, 10000, 10125, 10240, 10368
 RC_MIN_THREADS = 3
 
 
-def role_entry(role, n, t, seq, f, slot, names):
-    """A RoleInstance initialiser whose kernels fill `slot` of the instance."""
+def role_entry(role, n, t, seq, f, slot, names, start=0):
+    """A RoleInstance initialiser whose kernels fill `slot` of the instance, used from `start` workgroups."""
     slots = {"tile": "nullptr, nullptr", "rows": "nullptr, nullptr", "cols": "{nullptr, nullptr, nullptr, nullptr}",
              "real": "{nullptr, nullptr, nullptr, nullptr}", "rc": "{nullptr, nullptr}"}
     names = ", ".join(nm if nm == "nullptr" else f"(const void *)&{nm}" for nm in names)
@@ -310,7 +310,7 @@ def role_entry(role, n, t, seq, f, slot, names):
         p *= r
     assert p == n and elems_per_thread(n, seq, t) <= 40 and (f or 1) * t <= 1024, (n, t, seq)
     rs = ", ".join(str(r) for r in seq)
-    return f"    {{{role}, {f}, {{{n}, {t}, {len(seq)}, {{{rs}}}, {', '.join(slots.values())}}}}},"
+    return f"    {{{role}, {f}, {start}, {{{n}, {t}, {len(seq)}, {{{rs}}}, {', '.join(slots.values())}}}}},"
 
 
 def row_entries():
@@ -319,7 +319,8 @@ def row_entries():
         if n < ROWS_MIN or t < ROWS_MIN_THREADS or n in ROWS_TWO_PLANE:
             continue
         rs = ", ".join(str(r) for r in seq)
-        yield role_entry("ROLE_ROWS", n, t, seq, f, "rows", [f"stockham_rows_kernel<{w}, {n}, {t}, {sg}, {rs}>" for sg in (-1, 1)])
+        yield role_entry("ROLE_ROWS", n, t, seq, f, "rows", [f"stockham_rows_kernel<{w}, {n}, {t}, {sg}, {rs}>" for sg in (-1, 1)],
+                         ROW_FROM.get(n, 0))
 
 
 # Split-plane rows up to this length go through LDS in line order (planes.h), on the leaf's threads but for these:
@@ -376,7 +377,8 @@ def column_entries():
         rs = ", ".join(str(r) for r in seq)
         names = [f"stockham_cols_kernel<{w}, {n}, {t}, {sg}, {str(tw).lower()}, {rs}>" for sg in (-1, 1)]
         none = ["nullptr", "nullptr"]
-        yield role_entry("ROLE_COLS_TW" if tw else "ROLE_COLS", n, t, seq, f, "cols", none + names if tw else names + none)
+        start = LONG_COLUMN_FROM.get(n, 128) if n in LONG_COLUMN_SHAPES else (COLUMN_TW_FROM if tw else COLUMN_FROM).get(n, 0)
+        yield role_entry("ROLE_COLS_TW" if tw else "ROLE_COLS", n, t, seq, f, "cols", none + names if tw else names + none, start)
 
 
 def rc_entries():
@@ -384,7 +386,8 @@ def rc_entries():
         t, seq, w = ROWS_COLS_SHAPES.get(n, (t, seq, 0))
         if n <= COLUMN_LEAF_MAX and len(seq) >= 2 and t >= RC_MIN_THREADS:
             rs = ", ".join(str(r) for r in seq)
-            yield role_entry("ROLE_RC", n, t, seq, 0, "rc", [f"stockham_rc_kernel<{w}, {n}, {t}, {sg}, {rs}>" for sg in (-1, 1)])
+            yield role_entry("ROLE_RC", n, t, seq, 0, "rc", [f"stockham_rc_kernel<{w}, {n}, {t}, {sg}, {rs}>" for sg in (-1, 1)],
+                             ROWS_COLS_FROM.get(n, 0))
 
 
 # role files: name, header, entries, parts

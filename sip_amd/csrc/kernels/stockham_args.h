@@ -120,12 +120,14 @@ enum Role : int32_t {
     ROLE_COLS = 2,       // column tiles (columns.h)
     ROLE_COLS_TW = 3,    // column tiles with the four-step twiddle on store
     ROLE_RC = 4,         // rows in, columns out (rows_cols.h)
-    ROLE_PLANES = 5      // contiguous rows in two planes (planes.h); one direction, in rows_fwd
+    ROLE_PLANES = 5,     // contiguous rows in two planes (planes.h); one direction, in rows_fwd
+    ROLE_REAL_ODD = 6    // contiguous R2C / C2R rows of odd length (real_odd.h), in real_rows
 };
 
 struct RoleInstance {
     int32_t role;
-    int32_t F;  // transforms per workgroup; 0 = the planner's rule
+    int32_t F;     // transforms per workgroup; 0 = the planner's rule
+    int32_t from;  // workgroups from which it is used (fewer: the two-plane leaf, or the split of a long column)
     StockhamInstance inst;
 };
 

@@ -1,6 +1,8 @@
-"""Kernels whose threads and radices were chosen per role and length (column_shapes.py): every listed length
-against the FP64 oracle (rel-L2 2e-6), on counts that leave the last tile partly empty and, for columns,
-strides that do not fall on whole 128-byte lines."""
+"""Kernels whose threads and radices were chosen per role and length (column_shapes.py, row_shapes.py,
+real_shapes.py): every listed length against the FP64 oracle (rel-L2 2e-6), on counts that leave the last
+tile partly empty and, for columns, strides that do not fall on whole 128-byte lines. Columns and split
+stages run at two counts: few transforms (8-wide tiles, or the two-plane leaf where a shape needs many) and
+many (16-wide tiles, the listed shape)."""
 import importlib.util
 import os
 
@@ -34,36 +36,69 @@ def _vertical(n, b, direction):
     assert rel <= TOL
 
 
-@pytest.mark.parametrize("n", sorted(COLS.COLUMN_SHAPES) + [20, 24, 45])
+def _many(start):
+    """Columns that make more than 128 tiles of 16, and `start` of them, with a partly empty last one."""
+    return 16 * max(128, start) + 3
+
+
+def _check_role(st, n, shapes, start, few):
+    """The stage runs the listed shape (or the leaf where few transforms keep it) on the expected tile width."""
+    shape = shapes.get(n)
+    leaf = few and start > 0
+    assert st["L"] == n and st["split_lds"] == (0 if leaf else 1)
+    if shape and not leaf:
+        assert st["T"] == shape[0] and st["radices"] == shape[1]
+    if st["T"] >= 8:
+        assert st["F"] == 8 if few else (st["F"] % 16 == 0 or st["T"] > 64)
+
+
+@pytest.mark.parametrize("n", sorted(COLS.COLUMN_SHAPES) + [20, 24, 45, 400, 512, 1024])
 def test_column_shapes(torch_cuda, n):
-    _vertical(n, 37, INV if n % 3 else FWD)
+    start = COLS.COLUMN_FROM.get(n, 0)
+    for b, few in ((37, True), (_many(start), False)):
+        h = make([n], S.ASCEND_FFT_C2C, FWD, b, S.ASCEND_FFT_VERTICAL)
+        _check_role(h.describe()["stages"][0], n, COLS.COLUMN_SHAPES, start, few)
+        h.destroy()
+        _vertical(n, b, INV if n % 3 else FWD)
 
 
 @pytest.mark.parametrize("n", sorted(COLS.LONG_COLUMN_SHAPES))
 def test_long_column_shapes(torch_cuda, n):
-    """One pass from 128 tiles up (an odd count: 2051 columns), two below; both checked."""
-    h = make([n], S.ASCEND_FFT_C2C, FWD, 2051, S.ASCEND_FFT_VERTICAL)
-    assert h.describe()["fused"][0]["note"] == f"columns {n}"
+    """One pass from 128 tiles up, for some lengths later (an odd count, the last tile partly empty), two
+    below; both checked."""
+    width = COLS.LONG_COLUMN_SHAPES[n][3]
+    b = max(2051, width * COLS.LONG_COLUMN_FROM.get(n, 128) + 3)
+    h = make([n], S.ASCEND_FFT_C2C, FWD, b, S.ASCEND_FFT_VERTICAL)
+    f = h.describe()["fused"][0]
+    assert f["note"] == f"columns {n}" and f["F"] == width
     h.destroy()
-    _vertical(n, 2051, FWD if n % 2 else INV)
+    _vertical(n, b, FWD if n % 2 else INV)
     _vertical(n, 19, INV)
+
+
+def _split(n, first):
+    """The other factor: the shortest smooth leaf that makes a length which no single launch takes."""
+    m = next(v for v in S.smooth_lengths(33, 1024) if v * n > 32768)
+    return (n, m) if first else (m, n)
 
 
 @pytest.mark.parametrize("n", sorted(COLS.COLUMN_TW_SHAPES))
 def test_column_shapes_with_twiddle(torch_cuda, monkeypatch, n):
-    """First four-step stage of length n (forced factor), second stage the shortest smooth leaf that makes the
-    length one that no single launch takes."""
-    m = next(v for v in S.smooth_lengths(33, 1024) if v * n > 32768)
+    """First four-step stage of length n (forced factor)."""
+    _, m = _split(n, True)
     monkeypatch.setenv("SIP_FFT_SPLIT_L1", str(n))
     d = INV if n % 3 else FWD
-    x = oracle.uniform_complex((3, n * m), 0x5EED0F00 + n)
-    h = make([n * m], S.ASCEND_FFT_C2C, d, 3)
-    st = h.describe()["stages"][0]
-    assert st["L"] == n and st["tw4"] == n * m and st["T"] == COLS.COLUMN_TW_SHAPES[n][0]
-    h.destroy()
-    y = c2c(x, [n * m], d)
-    rel, _ = report(f"four-step {n} x {m}", y, oracle.c2c(x, sign_of(d)))
-    assert rel <= TOL
+    start = COLS.COLUMN_TW_FROM.get(n, 0)
+    for b, few in ((3, True), (_many(start) // m + 1, False)):
+        x = oracle.uniform_complex((b, n * m), 0x5EED0F00 + n)
+        h = make([n * m], S.ASCEND_FFT_C2C, d, b)
+        st = h.describe()["stages"][0]
+        h.destroy()
+        assert st["tw4"] == n * m
+        _check_role(st, n, COLS.COLUMN_TW_SHAPES, start, few and b * m <= 2048)
+        y = c2c(x, [n * m], d)
+        rel, _ = report(f"four-step {n} x {m} x {b}", y, oracle.c2c(x, sign_of(d)))
+        assert rel <= TOL
 
 
 def test_streaming_input_of_several_launches(torch_cuda):
@@ -81,7 +116,7 @@ ROWS = _shapes("row_shapes")
 
 @pytest.mark.parametrize("n", sorted(ROWS.ROW_SHAPES) + [25, 27, 35, 64, 66, 104, 117, 128, 16200])
 def test_row_shapes(torch_cuda, n):
-    b = max(3, min(75, (1 << 19) // n))
+    b = ROWS.ROW_FROM.get(n, max(3, min(75, (1 << 19) // n)))
     d = INV if n % 3 else FWD
     h = make([n], S.ASCEND_FFT_C2C, d, b)
     st = h.describe()["stages"][0]
@@ -159,16 +194,20 @@ def test_real_odd_lengths(torch_cuda, n):
 @pytest.mark.parametrize("n", sorted(REAL.ROWS_COLS_SHAPES))
 def test_rows_cols_shapes(torch_cuda, monkeypatch, n):
     """Second four-step stage of length n (the first factor forced)."""
-    m = next(v for v in S.smooth_lengths(33, 1024) if v * n > 32768)
+    m, _ = _split(n, False)
     monkeypatch.setenv("SIP_FFT_SPLIT_L1", str(m))
     d = INV if n % 3 else FWD
-    h = make([n * m], S.ASCEND_FFT_C2C, d, 3)
-    st = h.describe()["stages"][1]
-    h.destroy()
-    assert st["L"] == n and st["rc"] == 1 and st["T"] == REAL.ROWS_COLS_SHAPES[n][0]
-    x = oracle.uniform_complex((3, n * m), 0x5EED1400 + n)
-    rel, _ = report(f"four-step {m} x {n}", c2c(x, [n * m], d), oracle.c2c(x, sign_of(d)))
-    assert rel <= TOL
+    start = REAL.ROWS_COLS_FROM.get(n, 0)
+    for b, few in ((3, True), (_many(start) // m + 1, False)):
+        h = make([n * m], S.ASCEND_FFT_C2C, d, b)
+        st = h.describe()["stages"][1]
+        h.destroy()
+        assert st["L"] == n and st["rc"] == (0 if few and start else 1)
+        if not (few and start):
+            assert st["T"] == REAL.ROWS_COLS_SHAPES[n][0]
+        x = oracle.uniform_complex((b, n * m), 0x5EED1400 + n)
+        rel, _ = report(f"four-step {m} x {n} x {b}", c2c(x, [n * m], d), oracle.c2c(x, sign_of(d)))
+        assert rel <= TOL
 
 
 @pytest.mark.parametrize("n, factors", [(243000, [675, 360]), (327680, [640, 512]), (777600, [960, 810]),

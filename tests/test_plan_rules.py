@@ -54,3 +54,32 @@ def test_split_stages_cut_columns_alike():
     for n in (1080, 1200):
         st = S.describe_dry([n, 1024], C2C, FWD, 1)["stages"][1:]
         assert len(st) == 2 and [s["F"] for s in st] == [16, 16]
+
+
+@pytest.mark.parametrize("n,rows", [(12150, 257), (12960, 257), (14580, 257), (15000, 257), (16000, 320)])
+def test_row_shapes_of_few_rows(n, rows):
+    """Row shapes held to 64 registers need more workgroups than CUs; fewer rows run on the two-plane leaf."""
+    at = [S.describe_dry([n], C2C, FWD, b)["stages"][0]["split_lds"] for b in (1, rows - 1, rows, 4 * rows)]
+    assert at == [0, 0, 1, 1]
+
+
+@pytest.mark.parametrize("n", [729, 864, 972])
+def test_column_shapes_of_few_columns(n):
+    """The same for column shapes, from 385 tiles of 16; both run the same radices."""
+    few, last, many = (columns(n, b)["stages"][0] for b in (16, 6144, 6145))
+    assert [s["split_lds"] for s in (few, last, many)] == [0, 0, 1]
+    assert few["radices"] == last["radices"] == many["radices"]
+    assert S.describe_dry([n, 64], C2C, FWD, 4)["stages"][1]["split_lds"] == 0
+
+
+@pytest.mark.parametrize("n,first", [(1080, 128), (2048, 128), (1458, 320), (1728, 288), (1944, 320), (2025, 320)])
+def test_long_columns_from(n, first):
+    width = columns(n, 1 << 14)["fused"][0]["F"]
+    assert [len(columns(n, width * t)["fused"]) for t in (first - 1, first)] == [0, 1]
+
+
+@pytest.mark.parametrize("n", [2560, 3072, 4096])
+def test_long_columns_in_two_passes(n):
+    for b in (1024, 2048, 4096, 1 << 14):
+        d = columns(n, b)
+        assert d["fused"] == [] and len(d["stages"]) == 2
