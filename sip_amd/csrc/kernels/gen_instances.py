@@ -277,10 +277,19 @@ def instances():
 
 # Contiguous-row kernels (rows.h) from ROWS_MIN points up, with three or more threads per transform: shorter
 # rows, and leaves of fewer threads, are faster staged through LDS in line order (16: 5.3-6.0 TB/s staged,
-# 4.1 from their own threads). Three lengths are faster on the two-plane tile: 256 MiB of rows, single / two
-# planes, 15625 268 / 240 us, 15552 171 / 158; 8748 (512 rows 21.7 / 20.5, 700 rows 30.7 / 31.3).
+# 4.1 from their own threads). Leaves of 16 to 31 threads already read and write HBM from their own threads on
+# two planes; without a shape of their own one plane costs them its extra barriers (252 x 1 4.1 / 4.6 us, 351 x
+# 1024 6.6 / 7.3, 16 MiB of 325 11.2 / 12.2; 64 MiB within 5 % on average), except 125, 256 and 400 (256 x 32768
+# 27.7 / 21.7). Other lengths faster on the two-plane tile: 256 MiB of rows, single / two planes, 15625 268 / 240
+# us, 15552 171 / 158; 8748 (512 rows 21.7 / 20.5, 700 rows 30.7 / 31.3).
 ROWS_MIN, ROWS_MIN_THREADS = 24, 3
 ROWS_TWO_PLANE = {8748, 15552, 15625}
+ONE_PLANE_16 = {125, 256, 400}
+
+
+def two_plane_threads(n, t):
+    return 16 <= t < 32 and n not in ONE_PLANE_16
+
 
 # longest leaf used for column tiles (the host's kColumnLeafMax); every leaf up to it gets a column
 # kernel of its own (columns.h) with the shape measured for that role (column_shapes.py)
@@ -289,9 +298,12 @@ COLUMN_LEAF_MAX = 1024
 # with three or more threads (shorter ones are faster staged through LDS: 16 4.2 TB/s, from their own threads
 # 3.7), and those above where the single plane measured faster than the two-plane fused kernel on MI355X (R2C +
 # C2R of 256 MiB of reals, one box: 9216 155 / 211 us, 10000 161 / 226, 16384 131 / 173; it lost for most mixed
-# lengths from 12000 up, e.g. 15000 241 / 218, 13824 225 / 212)
+# lengths from 12000 up, e.g. 15000 241 / 218, 13824 225 / 212). Leaves of 16 to 31 threads without a shape take it
+# from 48 MiB on (R2C / C2R, two planes / one: 702 x 64 7.8 / 9.0, 7.9 / 8.0 us; 16 MiB of 750 16.4 / 17.1, 16.6 /
+# 17.7; 64 MiB of 750 43.7 / 39.4, 49.1 / 38.7).
 REAL_ROWS_MIN = 30
 REAL_ROWS_MAX = 8192
+REAL_FROM_POINTS = 6 << 20
 REAL_ROWS_LONG = {8640, 9000, 9216, 9375, 9600, 9720, 10000, 10125, 10240, 10368, 10800, 10935, 11250, 11664,
                   12288, 16384}
 # lengths up to COLUMN_LEAF_MAX with two or more passes and at least this many threads per transform also get
@@ -315,6 +327,8 @@ def role_entry(role, n, t, seq, f, slot, names, start=0):
 
 def row_entries():
     for n, t, seq in instances():
+        if n not in ROW_SHAPES and two_plane_threads(n, t):
+            continue
         t, seq, w, f = ROW_SHAPES.get(n, (t, seq, 0, 0))
         if n < ROWS_MIN or t < ROWS_MIN_THREADS or n in ROWS_TWO_PLANE:
             continue
@@ -349,11 +363,12 @@ def plane_entries():
 
 def real_row_entries():
     for n, t, seq in instances():
+        start = REAL_FROM_POINTS // n if n not in REAL_SHAPES and two_plane_threads(n, t) else 0
         t, seq, w, f = REAL_SHAPES.get(n, (t, seq, 0, 0))
         if t >= 3 and (REAL_ROWS_MIN <= n <= REAL_ROWS_MAX or n in REAL_ROWS_LONG):
             rs = ", ".join(str(r) for r in seq)
             yield role_entry("ROLE_REAL_ROWS", n, t, seq, f, "real", [
-                f"stockham_real_rows_kernel<{w}, {n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)])
+                f"stockham_real_rows_kernel<{w}, {n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)], start)
 
 
 # Odd lengths of the real transforms (real_odd.h), on the row kernels' shapes

@@ -167,9 +167,10 @@ def _real(n, b):
     assert rel <= TOL
 
 
-@pytest.mark.parametrize("L", sorted(REAL.REAL_SHAPES) + [32, 35, 64, 104, 128, 256])
+@pytest.mark.parametrize("L", sorted(REAL.REAL_SHAPES) + [32, 35, 64, 104, 128, 256, 162, 375])
 def test_real_shapes(torch_cuda, L):
-    b = max(3, min(75, (1 << 18) // L))
+    """162 and 375: leaves of 16 to 31 threads, on one plane from 48 MiB."""
+    b = (6 << 20) // L + 1 if L in (162, 375) else max(3, min(75, (1 << 18) // L))
     h = make([2 * L], S.ASCEND_FFT_R2C, FWD, b)
     st = h.describe()["stages"][0]
     h.destroy()

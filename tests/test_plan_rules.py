@@ -83,3 +83,18 @@ def test_long_columns_in_two_passes(n):
     for b in (1024, 2048, 4096, 1 << 14):
         d = columns(n, b)
         assert d["fused"] == [] and len(d["stages"]) == 2
+
+
+@pytest.mark.parametrize("n,one", [(162, 0), (252, 0), (288, 0), (360, 0), (375, 0), (8748, 0), (125, 1), (256, 1), (300, 1),
+                                   (400, 1), (104, 1), (500, 1)])
+def test_rows_on_one_or_two_planes(n, one):
+    """Leaves of 16 to 31 threads keep the two-plane tile unless one plane was measured faster."""
+    for b in (1, 64, 4096):
+        assert S.describe_dry([n], C2C, FWD, b)["stages"][0]["split_lds"] == one
+
+
+@pytest.mark.parametrize("n,start", [(250, 0), (324, (6 << 20) // 162), (750, (6 << 20) // 375), (512, 0), (4096, 0)])
+def test_real_rows_on_one_or_two_planes(n, start):
+    for t in (S.ASCEND_FFT_R2C, S.ASCEND_FFT_C2R):
+        at = [S.describe_dry([n], t, FWD, b)["stages"][0]["split_lds"] for b in (1, max(1, start - 1), max(1, start))]
+        assert at == ([0, 0, 1] if start else [1, 1, 1])
