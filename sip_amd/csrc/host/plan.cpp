@@ -1034,6 +1034,14 @@ struct Builder {
         if (F >= 16) F &= ~15;
         const int64_t least = q.nfft <= kColumnLeafMax ? 2 : 4;
         if (least * (F - a.halo) < F) return;
+        // Stages where the one launch does not pay. Below 640K points, frames that do not overlap, or hardly do on few
+        // threads: a tile's threads sum their samples in long chains (staged / one launch: hop = n, 24 x 2049 frames 8.2 /
+        // 13.3 us, 256 x 9 7.1 / 11.4, 400 x 64 9.1 / 17.6, 640 x 4 x 200 14.2 / 17.1, but 160 x 2 x 2049 17.0 / 15.5; hop =
+        // n / 2, 24 x 2049 8.3 / 10.1, 80 x 4 x 200 10.2 / 13.2). And a handful of long frames (1000, hop 125, 2 frames
+        // 9.5 / 14.8).
+        const int64_t total = q.frames * q.channel;
+        const bool long_sums = a.halo < (ii->T < 8 ? 2 : 1) && total * q.nfft < 5 * (int64_t(1) << 17);
+        if ((long_sums || (total < 8 && q.nfft >= 384)) && !fusing_always()) return;
         // Few frames: smaller tiles while there are fewer than two per CU, or, where the half tile reads its frames
         // more than one and a half times, than half as many as CUs. Measured on MI355X, frames per tile: 1440, hop
         // 720, 164 frames 11 / 8 / 4 / 2 18.9 / 15.5 / 11.8 / 11.7 us, 4 channels 20.4 / 17.0 / 13.5 / 14.8, 16 channels

@@ -431,6 +431,10 @@ def write_roles(outdir):
 # One-launch inverse short-time transforms (istft.h): every 2,3,5-smooth frame length in this range,
 # with the leaf's radix sequence and threads.
 ISTFT_MIN, ISTFT_MAX, ISTFT_PARTS = 24, 1499, 6
+# Lengths whose kernel spilled 40 to 116 bytes a lane when held to 64 registers (two 1024-thread tiles per CU);
+# within 73 to 91 it does not (64 MiB, held / free: 320, hop 40 68.8 / 46.5 us, 640, hop 160 64.5 / 39.2, 40, hop 5 65.2
+# / 29.4). Others that spill less keep the limit (1000, hop 250 48.2 / 60.5; 500, hop 62 46.6 / 54.0).
+ISTFT_FREE = {40, 45, 60, 160, 180, 192, 240, 320, 400, 640, 800}
 
 
 def istft_instances():
@@ -452,7 +456,7 @@ def write_istft(outdir):
         items = inst[k::ISTFT_PARTS]
         for n, t, seq in items:
             rs = ", ".join(str(r) for r in seq)
-            lines.append(f"    {{{n}, {t}, {len(seq)}, {{{rs}}}, (const void *)&istft_kernel<{n}, {t}, {rs}>}},")
+            lines.append(f"    {{{n}, {t}, {len(seq)}, {{{rs}}}, (const void *)&istft_kernel<{0 if n in ISTFT_FREE else 8}, {n}, {t}, {rs}>}},")
         lines += ["};", f"extern const int g_istft_part_{k}_count = {len(items)};", "}  // namespace sip"]
         write_if_changed(os.path.join(outdir, f"istft_part_{k}.hip"), "\n".join(lines) + "\n")
     inc = ["// Generated by gen_instances.py (do not edit)."] + [f"SIP_ISTFT_PART({k})" for k in range(ISTFT_PARTS)]

@@ -14,6 +14,9 @@
 // launch: 8 channels x 2049 frames of 1024, hop 256 126.5 / 67.7 us; 4 channels, 2^23 points in all:
 // 256, hop 64 53 / 32 us, 400, hop 100 69 / 34, 1000, hop 250 83 / 47, 1200, hop 300 223 / 55.
 //
+// W: waves per SIMD the register budget is held to (8: 64 registers, two 1024-thread tiles per CU; 0: the
+// compiler's choice, for the lengths that would spill, gen_instances.py).
+//
 // The sums run in the order, and with the operations, of the staged overlap-add (aux.hip). LDS: one
 // plane, the real parts of all frames summed first, then the imaginary parts.
 #pragma once
@@ -31,8 +34,8 @@ struct LastRadix<R> {
     static constexpr int value = R;
 };
 
-template <int L, int T, int... Rs>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void istft_kernel(const IstftArgs a)
+template <int W, int L, int T, int... Rs>
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(W))) void istft_kernel(const IstftArgs a)
 {
     extern __shared__ float pl[];
     constexpr int R0 = first_of<Rs...>(), NBF0 = L / R0, NB0 = (NBF0 + T - 1) / T;

@@ -131,6 +131,25 @@ def test_istft_one_launch(torch_cuda, monkeypatch, ch, n, hop, frames):
     _agree(f"istft ch={ch} n={n} hop={hop} frames={frames}", got, staged, oracle.istft(x, n, hop, w), 2e-6)
 
 
+@pytest.mark.parametrize("n", [40, 45, 60, 160, 180, 192, 240, 320, 400, 640, 800])
+def test_istft_lengths_off_the_register_limit(torch_cuda, monkeypatch, n):
+    test_istft_one_launch(torch_cuda, monkeypatch, 2, n, n // 4, 90)
+
+
+@pytest.mark.parametrize("ch,n,hop,frames,fused", [(1, 24, 24, 64, 0), (1, 400, 400, 64, 0), (4, 640, 640, 200, 0),
+                                                   (2, 160, 160, 2049, 1), (4, 80, 40, 200, 0), (4, 128, 64, 200, 1),
+                                                   (1, 1000, 125, 2, 0), (1, 1000, 125, 9, 1), (8, 1024, 256, 40, 1)])
+def test_istft_route(torch_cuda, monkeypatch, ch, n, hop, frames, fused):
+    """Where the stages are faster the plan keeps them."""
+    import torch
+    monkeypatch.delenv("SIP_FFT_FUSE", raising=False)
+    h = S.FftHandle()
+    x = torch.empty(ch, n, frames, dtype=torch.complex64, device="cuda")
+    assert h.istft_make_plan(x, n, hop, n) == S.ACL_SUCCESS
+    assert len(h.describe()["fused"]) == fused
+    h.destroy()
+
+
 @pytest.mark.parametrize("mode", [S.PREC_F16_SPLIT, S.PREC_BF16_SPLIT3])
 @pytest.mark.parametrize("a, b, batch", [(2048, 525, 4), (1536, 1050, 2)])
 def test_precision_long_columns(torch_cuda, monkeypatch, a, b, batch, mode):
