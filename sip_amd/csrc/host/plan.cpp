@@ -1407,12 +1407,14 @@ void plan_materialize_external(Plan &p, const std::vector<const int64_t *> &dev_
 // 2D 1024^2 x 128 855 -> 837 us, 3D 128^3 x 64 801 -> 786 us, 32768 x 4096 540 -> 532 us, but
 // slower on inputs that the last-level cache still holds (2000 x 8192 45 -> 56 us, R2C 8192 x 4096
 // 48 -> 52 us, four-step 43200 x 1056 341 -> 359 us, batching workload 8.9 -> 9.3 ms), hence the
-// size threshold. A plan of several launches loads its input nontemporally already when what one
-// execution touches (input, intermediates, output) is more than half of that cache: the input is most
-// likely not in it (a program's other data between two calls is as large), and loading it past the cache
-// keeps the intermediate there for the next launch. On three buffer sets in turn / on one set over and
-// over, cached -> nontemporal: 1048576 x 8 72.6 -> 54.2 / 53.3 -> 54.9 us, 65536 x 128 54.7 -> 50.3 / 47.9 ->
-// 52.0, 1000000 x 8 85.0 -> 78.4 / 77.5 -> 78.0, 100000 x 83 74.2 -> 70.0 / 65.7 -> 69.9.
+// size threshold. A plan of several launches whose first stage walks columns of 1000 points or more in whole lines
+// loads its input nontemporally already when what one execution touches (input, intermediates, output) is more than
+// half of that cache: two such tiles per CU read more than the intermediate can share the cache with. us on three
+// buffer sets in turn / on one set over and over / on one set that the kernel before writes (both kernels), cached ->
+// nontemporal: 1048576 x 8 70.9 -> 53.3 / 52.9 -> 54.5 / 61.3 -> 61.2, 1024000 x 8 71.8 -> 63.9 / 62.8 -> 63.4 / 72.3 ->
+// 71.2. Shorter first stages and rows keep cached loads: what they gain on cold inputs (65536 x 128 54.4 -> 50.6, 1024^2
+// x 16 101.6 -> 95.0) they lose on the inputs of a program that has just written or read them (46.7 -> 51.2, 90.9 ->
+// 95.5), half lines more (40000 x 220 after a pass over its input 71.8 -> 86.1).
 void plan_mark_streaming(Plan &p)
 {
     const bool on_out = env_flag("SIP_FFT_NT_OUT", true), on_in = env_flag("SIP_FFT_NT_IN", true);
@@ -1458,7 +1460,7 @@ void plan_mark_streaming(Plan &p)
         s.sa.nt_out = (on_out && !read_later && aligned_out) ? 1 : 0;
         const int64_t in_bytes = s.sa.nfft * (int64_t)s.sa.in_len * 8;
         const bool cold = i == 0 && run.size() > 1 && s.in.kind == BUF_IN && !gathered && footprint > kNtInFootprint &&
-                          (!cols_in || s.sa.tin.es % 8 == 0);
+                          cols_in && s.sa.tin.es % 16 == 0 && s.sa.in_len >= 1000;
         s.sa.nt_in = (on_in && s.sa.io_mode == IO_C2C && (in_bytes >= kNtInBytes || cold) && aligned_in) ? 1 : 0;
     }
 }
