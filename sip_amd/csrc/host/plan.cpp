@@ -483,11 +483,12 @@ struct Builder {
         // pass straight from / to HBM), unless the tuner or SIP_FFT_SPLIT_LDS=0 asks for the two-plane leaf.
         const bool flat_in = tin.es == 1 && !tin.unit_f && !in_sep, flat_out = tout.es == 1 && !tout.unit_f && !out_sep;
         const int64_t nfft = count(normalize(in.dims));
-        // A shape that needs many workgroups: gathered groups have other launches beside them, and where the
-        // arithmetic must not depend on the number of transforms (!p.big_leaf) the leaf is for all.
+        // A shape for many or for not too many transforms: gathered groups have other launches beside them, and where the
+        // arithmetic must not depend on the number of transforms (!p.big_leaf) a shape for many is for none.
         auto enough = [&](const RoleInstance *r, int64_t width) {
-            if (!r || r->from == 0) return true;
-            return p.big_leaf && (tin.tab_dim >= 0 || nfft >= (r->from - 1) * width + 1);
+            if (!r || tin.tab_dim >= 0) return !r || r->from == 0 || p.big_leaf;
+            if (!p.big_leaf) return r->from == 0;
+            return (r->from == 0 || nfft >= (r->from - 1) * width + 1) && (r->to == 0 || nfft <= r->to);
         };
         const RoleInstance *role = nullptr;
         if (columns && !mf && split_columns(L)) {

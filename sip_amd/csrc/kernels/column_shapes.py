@@ -104,6 +104,10 @@ COLUMN_TW_SHAPES = {
 
 # as COLUMN_FROM
 COLUMN_TW_FROM = {625: 257, 729: 257, 972: 257}
+# Points up to which a shape is used: with two tiles per CU the input and the intermediate share the last-level cache,
+# which beyond 96 MiB of each costs more than the overlap gains (two-plane leaf / shape: 995328 x 16 as 972 x 1024 146 /
+# 165 us, 1000000 x 16 167 / 185, x 32 330 / 351, 1024000 x 32 297 / 326; 1000000 x 8 87 / 79).
+COLUMN_TW_POINTS = {972: 12 << 20, 1000: 12 << 20}
 
 # Whole axes above 1024 points in one pass (no four-step twiddle), with the columns per tile: 16 columns
 # take 32 values per thread (waves per SIMD 4: 128 registers, one workgroup per CU), 8 fewer but half

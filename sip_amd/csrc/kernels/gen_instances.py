@@ -15,7 +15,8 @@ import os
 import sys
 
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))  # also when loaded from a path
-from column_shapes import COLUMN_FROM, COLUMN_SHAPES, COLUMN_TW_FROM, COLUMN_TW_SHAPES, LONG_COLUMN_FROM, LONG_COLUMN_SHAPES
+from column_shapes import (COLUMN_FROM, COLUMN_SHAPES, COLUMN_TW_FROM, COLUMN_TW_POINTS, COLUMN_TW_SHAPES, LONG_COLUMN_FROM,
+                           LONG_COLUMN_SHAPES)
 from real_shapes import REAL_SHAPES, ROWS_COLS_FROM, ROWS_COLS_SHAPES
 from row_shapes import ROW_FROM, ROW_SHAPES
 from split_rates import SPLIT_RATES
@@ -284,6 +285,10 @@ def instances():
 # us, 15552 171 / 158; 8748 (512 rows 21.7 / 20.5, 700 rows 30.7 / 31.3).
 ROWS_MIN, ROWS_MIN_THREADS = 24, 3
 ROWS_TWO_PLANE = {8748, 15552, 15625}
+# Leaves of fewer than 16 threads without a shape lose on one plane from 64 MiB on, where their narrow runs bound
+# them: two planes in line order / one, 48 x 349525 57.3 / 68.8 us, x 1398101 193 / 252, 33 x 508400 61.3 / 72.5, 27, 28,
+# 32, 39, 42, 44, 50 .. 56, 66, 75, 78, 84 and 128 3 to 28 %; below 48 MiB they win (48 x 21845 12.4 / 9.4).
+ROWS_POINTS = {n: 6 << 20 for n in (27, 28, 32, 33, 39, 42, 44, 48, 50, 52, 54, 56, 66, 75, 78, 84, 128)}
 ONE_PLANE_16 = {125, 256, 400}
 
 
@@ -304,6 +309,9 @@ COLUMN_LEAF_MAX = 1024
 REAL_ROWS_MIN = 30
 REAL_ROWS_MAX = 8192
 REAL_FROM_POINTS = 6 << 20
+# as ROWS_POINTS (R2C / C2R, two planes / one: 66 x 508400 68.9 / 96.9, 70.3 / 91.3 us; 84 x 399457 1.11, 1.18)
+REAL_POINTS = {n: 6 << 20 for n in (35, 42, 44, 50, 52, 54, 55, 56, 65, 66, 70, 75, 78, 84, 110, 112)}
+REAL_POINTS.update({33: 2 << 20, 39: 2 << 20})
 REAL_ROWS_LONG = {8640, 9000, 9216, 9375, 9600, 9720, 10000, 10125, 10240, 10368, 10800, 10935, 11250, 11664,
                   12288, 16384}
 # lengths up to COLUMN_LEAF_MAX with two or more passes and at least this many threads per transform also get
@@ -311,8 +319,9 @@ REAL_ROWS_LONG = {8640, 9000, 9216, 9375, 9600, 9720, 10000, 10125, 10240, 10368
 RC_MIN_THREADS = 3
 
 
-def role_entry(role, n, t, seq, f, slot, names, start=0):
-    """A RoleInstance initialiser whose kernels fill `slot` of the instance, used from `start` workgroups."""
+def role_entry(role, n, t, seq, f, slot, names, start=0, points=0):
+    """A RoleInstance initialiser whose kernels fill `slot` of the instance, used from `start` workgroups
+    and up to `points` points (0: any number)."""
     slots = {"tile": "nullptr, nullptr", "rows": "nullptr, nullptr", "cols": "{nullptr, nullptr, nullptr, nullptr}",
              "real": "{nullptr, nullptr, nullptr, nullptr}", "rc": "{nullptr, nullptr}"}
     names = ", ".join(nm if nm == "nullptr" else f"(const void *)&{nm}" for nm in names)
@@ -322,7 +331,7 @@ def role_entry(role, n, t, seq, f, slot, names, start=0):
         p *= r
     assert p == n and elems_per_thread(n, seq, t) <= 40 and (f or 1) * t <= 1024, (n, t, seq)
     rs = ", ".join(str(r) for r in seq)
-    return f"    {{{role}, {f}, {start}, {{{n}, {t}, {len(seq)}, {{{rs}}}, {', '.join(slots.values())}}}}},"
+    return f"    {{{role}, {f}, {start}, {points // n}, {{{n}, {t}, {len(seq)}, {{{rs}}}, {', '.join(slots.values())}}}}},"
 
 
 def row_entries():
@@ -334,7 +343,7 @@ def row_entries():
             continue
         rs = ", ".join(str(r) for r in seq)
         yield role_entry("ROLE_ROWS", n, t, seq, f, "rows", [f"stockham_rows_kernel<{w}, {n}, {t}, {sg}, {rs}>" for sg in (-1, 1)],
-                         ROW_FROM.get(n, 0))
+                         ROW_FROM.get(n, 0), ROWS_POINTS.get(n, 0))
 
 
 # Split-plane rows up to this length go through LDS in line order (planes.h), on the leaf's threads but for these:
@@ -368,7 +377,8 @@ def real_row_entries():
         if t >= 3 and (REAL_ROWS_MIN <= n <= REAL_ROWS_MAX or n in REAL_ROWS_LONG):
             rs = ", ".join(str(r) for r in seq)
             yield role_entry("ROLE_REAL_ROWS", n, t, seq, f, "real", [
-                f"stockham_real_rows_kernel<{w}, {n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)], start)
+                f"stockham_real_rows_kernel<{w}, {n}, {t}, {sg}, {m}, {rs}>" for m in (1, 2) for sg in (-1, 1)], start,
+                             REAL_POINTS.get(n, 0))
 
 
 # Odd lengths of the real transforms (real_odd.h), on the row kernels' shapes
@@ -393,7 +403,8 @@ def column_entries():
         names = [f"stockham_cols_kernel<{w}, {n}, {t}, {sg}, {str(tw).lower()}, {rs}>" for sg in (-1, 1)]
         none = ["nullptr", "nullptr"]
         start = LONG_COLUMN_FROM.get(n, 128) if n in LONG_COLUMN_SHAPES else (COLUMN_TW_FROM if tw else COLUMN_FROM).get(n, 0)
-        yield role_entry("ROLE_COLS_TW" if tw else "ROLE_COLS", n, t, seq, f, "cols", none + names if tw else names + none, start)
+        yield role_entry("ROLE_COLS_TW" if tw else "ROLE_COLS", n, t, seq, f, "cols", none + names if tw else names + none, start,
+                         COLUMN_TW_POINTS.get(n, 0) if tw else 0)
 
 
 def rc_entries():

@@ -128,6 +128,7 @@ struct RoleInstance {
     int32_t role;
     int32_t F;     // transforms per workgroup; 0 = the planner's rule
     int32_t from;  // workgroups from which it is used (fewer: the two-plane leaf, or the split of a long column)
+    int32_t to;    // transforms up to which it is used (more: the two-plane leaf); 0 = any number
     StockhamInstance inst;
 };
 

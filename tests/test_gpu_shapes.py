@@ -129,6 +129,16 @@ def test_row_shapes(torch_cuda, n):
     assert rel <= TOL
 
 
+@pytest.mark.parametrize("n", sorted(_shapes("gen_instances").ROWS_POINTS))
+def test_short_rows_of_many(torch_cuda, n):
+    """On both sides of the count from which short rows go through LDS in line order."""
+    points = _shapes("gen_instances").ROWS_POINTS[n]
+    for b in (points // n, points // n + 1):
+        x = oracle.uniform_complex((b, n), 0x5EED1600 + n)
+        rel, _ = report(f"rows {n} x {b}", c2c(x, [n], INV if n % 2 else FWD), oracle.c2c(x, sign_of(INV if n % 2 else FWD)))
+        assert rel <= TOL
+
+
 @pytest.mark.parametrize("n", [2, 3, 7, 8, 11, 13, 16, 20, 22, 24, 25, 26, 30, 33, 39, 40, 45, 48, 50, 52, 54, 56, 64, 65, 66, 81,
                                100, 104, 200,
                                243, 300, 1000, 1200, 3600, 4096, 15000, 15625, 16384])

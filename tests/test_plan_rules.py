@@ -106,3 +106,28 @@ def test_real_rows_on_one_or_two_planes(n, start):
 def test_streaming_inputs(dims, b, nt):
     """Below 512 MiB only long first-stage columns in whole lines pass the last-level cache."""
     assert S.describe_dry(dims, C2C, FWD, b)["stages"][0]["nt_in"] == nt
+
+
+@pytest.mark.parametrize("n,points", [(27, 6 << 20), (48, 6 << 20), (50, 6 << 20), (128, 6 << 20), (64, 0), (100, 0), (104, 0)])
+def test_short_rows_of_many(n, points):
+    """Leaves of fewer than 16 threads that lose on one plane at large sizes leave it there."""
+    for b in (1, 64, max(1, points // n) if points else 1 << 20):
+        assert S.describe_dry([n], C2C, FWD, b)["stages"][0]["split_lds"] == 1
+    if points:
+        assert S.describe_dry([n], C2C, FWD, points // n + 1)["stages"][0]["split_lds"] == 0
+
+
+@pytest.mark.parametrize("n,points", [(66, 2 << 20), (100, 6 << 20), (84, 6 << 20), (128, 0)])
+def test_short_real_rows_of_many(n, points):
+    for t in (S.ASCEND_FFT_R2C, S.ASCEND_FFT_C2R):
+        b = points // (n // 2) if points else 1 << 20
+        assert S.describe_dry([n], t, FWD, b)["stages"][0]["split_lds"] == 1
+        if points:
+            assert S.describe_dry([n], t, FWD, b + 1)["stages"][0]["split_lds"] == 0
+
+
+@pytest.mark.parametrize("n,last", [(995328, 12), (1000000, 12), (1024000, 12)])
+def test_long_first_stages_of_many(n, last):
+    """972- and 1000-point first stages keep two tiles per CU up to 96 MiB."""
+    at = [S.describe_dry([n], C2C, FWD, b)["stages"][0]["split_lds"] for b in (8, last, last + 1, 32)]
+    assert at == [1, 1, 0, 0]
