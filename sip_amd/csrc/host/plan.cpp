@@ -1431,6 +1431,15 @@ void plan_mark_streaming(Plan &p)
         if (run[i]->in.kind != run[i]->out.kind || run[i]->in.ws_index != run[i]->out.ws_index)
             footprint += a.nfft * (int64_t)a.out_len * 8;
     }
+    // Launches of one array in one order: where a 2D / 3D transform outgrows the last-level cache, a column launch in
+    // XCD order after rows in launch order finds less of what they left. In launch order throughout / mixed / XCD order
+    // throughout, 128 MiB: 243 x 60 x 1150 124 / 133 / 114 us, 300 x 486 x 115 127 / 134 / 116, 500 x 1250 x 26 132 / 143 /
+    // 133, 36 x 96 x 60 x 80 162 / 175 / 156; 64 MiB lose 3 % by it on average.
+    const bool in_xcd_order = std::any_of(run.begin(), run.end(), [](const Stage *s) { return s->sa.xcd_remap != 0; });
+    if (in_xcd_order && p.fftType == kTypeC2C && p.sizes.size() > 1 && !gathered && footprint > (int64_t(192) << 20) &&
+        p.tune.xcd < 0 && !std::getenv("SIP_FFT_XCD"))
+        for (Stage *s : run)
+            if (s->kind == StageKind::Stockham) s->sa.xcd_remap = 1;
     for (size_t i = 0; i < run.size(); i++) {
         Stage &s = *run[i];
         if (s.kind != StageKind::Stockham) continue;

@@ -131,3 +131,9 @@ def test_long_first_stages_of_many(n, last):
     """972- and 1000-point first stages keep two tiles per CU up to 96 MiB."""
     at = [S.describe_dry([n], C2C, FWD, b)["stages"][0]["split_lds"] for b in (8, last, last + 1, 32)]
     assert at == [1, 1, 0, 0]
+
+
+@pytest.mark.parametrize("dims,b,order", [([243, 60], 1150, [1, 1]), ([500, 1250], 26, [1, 1]), ([36, 96, 60], 80, [1, 1, 1]),
+                                          ([243, 60], 288, [0, 1]), ([512, 1296], 25, [0, 0]), ([243, 60], 2300, [1, 1])])
+def test_launches_of_one_array_in_one_order(dims, b, order):
+    assert [s["xcd_remap"] for s in S.describe_dry(dims, C2C, FWD, b)["stages"]] == order
