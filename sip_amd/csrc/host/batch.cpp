@@ -185,6 +185,34 @@ void store_cache(const std::string &key, const Tune &t)
 
 // ------------------------------------------------------------------ group plans
 
+// Whether a problem's output lies on an input of the group, other than an in-place problem's on its own: stages
+// read all inputs of a Bluestein group before they write, one launch does not.
+bool outputs_on_inputs(const BatchPlan &bp, const Group &g)
+{
+    std::vector<std::pair<uintptr_t, uintptr_t>> ins;  // begin, end
+    auto size = [&](int i) { return (uintptr_t)(bp.batches[(size_t)i] * g.n * 8); };
+    uintptr_t longest = 0;
+    for (int i : g.members) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(bp.ins[(size_t)i]);
+        ins.emplace_back(a, a + size(i));
+        longest = std::max(longest, size(i));
+    }
+    std::sort(ins.begin(), ins.end());
+    for (int i : g.members) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(bp.outs[(size_t)i]), b = a + size(i);
+        const bool in_place = bp.ins[(size_t)i] == bp.outs[(size_t)i];
+        // inputs that begin before b and may reach beyond a
+        auto it = std::lower_bound(ins.begin(), ins.end(), std::make_pair(a > longest ? a - longest : 0, uintptr_t(0)));
+        bool own = in_place;  // the problem's own input, once
+        for (; it != ins.end() && it->first < b; ++it) {
+            if (it->second <= a) continue;
+            if (!own || it->first != a || it->second != b) return true;
+            own = false;
+        }
+    }
+    return false;
+}
+
 std::unique_ptr<Plan> build_group_plan(const BatchPlan &bp, const Group &g, const Tune &t)
 {
     auto p = std::make_unique<Plan>();
@@ -208,6 +236,7 @@ std::unique_ptr<Plan> build_group_plan(const BatchPlan &bp, const Group &g, cons
             out_rows.push_back(ob + r * g.n);
         }
     }
+    p->fuse = !outputs_on_inputs(bp, g);
     plan_build_gathered_c2c(*p, g.n, in_rows, out_rows, reinterpret_cast<void *>(in_lo),
                             reinterpret_cast<void *>(out_lo));
     plan_materialize(*p);

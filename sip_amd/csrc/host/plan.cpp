@@ -922,7 +922,7 @@ struct Builder {
             add_stockham(L, sign, in, out, IO_C2C, L, L, 0, 1, "columns " + std::to_string(L), true);
             Stage st = std::move(p.stages.back());
             p.stages.pop_back();
-            p.fusions.push_back(Fusion{first, last, std::move(st)});
+            fuse(first, last, std::move(st));
         }
     }
 
@@ -945,8 +945,18 @@ struct Builder {
         fuse_bluestein(first, N, sign, in, out);
     }
 
-    // The stages from `first` to the last one run as one launch of `st`'s kernel.
-    void fuse(size_t first, Stage &&st) { p.fusions.push_back(Fusion{first, p.stages.size() - 1, std::move(st)}); }
+    // The stages first .. last run as the one launch `st`.
+    void fuse(size_t first, size_t last, Stage &&st)
+    {
+        // the first stage of a split, of a chirp-z convolution and of an ISTFT writes an array as large as its input
+        if (st.in.kind == BUF_IN && st.out.kind == BUF_OUT) {
+            const BufRef &w = p.stages[first].out;
+            if (w.kind != BUF_WS)
+                throw SipError(AsdSip::ACL_ERROR_INTERNAL_ERROR, "fused launch over stages without a workspace");
+            st.spare_ws = w.ws_index;
+        }
+        p.fusions.push_back(Fusion{first, last, std::move(st)});
+    }
 
     // One-launch Bluestein (kernels/bluestein.h) for every length whose convolution fits an
     // instance (N <= 16384), any strides; the precision form keeps its matrix-core FFT stages. The longest
@@ -956,7 +966,7 @@ struct Builder {
     void fuse_bluestein(size_t first, int64_t N, int sign, const Lay &in, const Lay &out)
     {
         const BluesteinInstance *bi = p.precision == PREC_FP32 ? find_bluestein_instance(2 * N - 1) : nullptr;
-        if (!bi || !fusing()) return;
+        if (!bi || !fusing() || !p.fuse) return;
         bool ok = true;
         Stage st;
         st.kind = StageKind::Stockham;
@@ -1003,7 +1013,7 @@ struct Builder {
         st.block = dim3((unsigned)(F * T));
         st.lds = (size_t)(F * per);
         st.note = "bluestein " + std::to_string(N) + " on " + std::to_string(bi->M) + " points";
-        fuse(first, std::move(st));
+        fuse(first, p.stages.size() - 1, std::move(st));
     }
 
     // One-launch inverse short-time transform (kernels/istft.h): 2,3,5-smooth frame lengths whose
@@ -1066,7 +1076,7 @@ struct Builder {
         st.block = dim3((unsigned)(F * ii->T));
         st.lds = (size_t)F * a.LP * 4;
         st.note = "istft " + std::to_string(q.nfft) + ", hop " + std::to_string(q.hop);
-        fuse(first, std::move(st));
+        fuse(first, p.stages.size() - 1, std::move(st));
     }
 
     // Real-to-complex transform of the last axis (n reals -> n/2+1 bins per row).
@@ -1568,8 +1578,34 @@ void plan_execute_istft(Plan &p, const void *in, const float *window, void *out)
     plan_execute(p, in, out);
 }
 
+// Copies the caller's input into the fused launch's workspace array where storing outputs could overwrite inputs
+// that other workgroups still read: the buffers overlap, and are not one array transformed in place (there every
+// transform stays where it was).
+static void step_aside(Plan &p, const void *&in, const void *&in_im, const void *out, const void *out_im)
+{
+    if (p.launches.empty() || p.launches[0]->spare_ws < 0) return;
+    const bool istft = p.istft.active;
+    int64_t n_in = p.batch, n_out;
+    for (int64_t d : p.sizes) n_in *= d;
+    n_out = istft ? p.istft.channel * p.istft.out_len : n_in;
+    const size_t esz = in_im ? 4 : 8, bytes = (size_t)n_in * esz;
+    auto clash = [&](const void *a, const void *b) {
+        const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+        return (x != y || istft) && x < y + (size_t)n_out * esz && y < x + bytes;
+    };
+    bool any = clash(in, out);
+    if (in_im) any = any || clash(in, out_im) || clash(in_im, out) || clash(in_im, out_im);
+    if (!any) return;
+    char *w = static_cast<char *>(p.workspace) + p.ws_offsets[(size_t)p.launches[0]->spare_ws];
+    SIP_HIP_CHECK(hipMemcpyAsync(w, in, bytes, hipMemcpyDeviceToDevice, p.stream));
+    if (in_im) SIP_HIP_CHECK(hipMemcpyAsync(w + bytes, in_im, bytes, hipMemcpyDeviceToDevice, p.stream));
+    in = w;
+    if (in_im) in_im = w + bytes;
+}
+
 void plan_execute_sep(Plan &p, const void *in, const void *in_im, void *out, void *out_im)
 {
+    step_aside(p, in, in_im, out, out_im);
     // imaginary planes of the user buffers (split-plane plans only)
     auto im_of = [&](const BufRef &b) -> float * {
         if (b.kind == BUF_IN) return static_cast<float *>(const_cast<void *>(in_im));

@@ -97,6 +97,10 @@ struct Stage {
     IstftArgs ia{};
     // Kernel of a launch that stands for several stages (Plan::fusions); null for a stage of its own
     const void *fused_fn = nullptr;
+    // Fused launch from the caller's input to the caller's output: a workspace array of the stages it stands for, at
+    // least as large as the input. Those had read all of the input before the first output was written; the launch
+    // takes the input from there where the caller's buffers overlap (plan_execute). -1: no such launch.
+    int spare_ws = -1;
     std::string note;
 };
 
@@ -142,6 +146,8 @@ struct Plan {
     // Transforms per launch from which those leaves replace the split; 0 takes the plain-plan
     // default (256). The batching form's groups run concurrently on several chains and set 64.
     int64_t big_leaf_rows = 0;
+    // False: every stage on its own (gathered rows some of whose outputs lie on other rows' inputs)
+    bool fuse = true;
     // ISTFT plan (asdFftIstftMakePlan): inverse C2C of the (channel, n_fft, frames) spectra into a
     // frame workspace, then the windowed overlap-add into (channel, out_len)
     struct Istft {
