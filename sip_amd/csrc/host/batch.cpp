@@ -114,12 +114,14 @@ std::string device_name()
     return prop.gcnArchName;
 }
 
+// A saved choice holds for the kernels (kernel_set) and the planner's rules (the number in front, raised with them)
+// that it was timed with.
 std::string tune_key(int64_t n, int64_t rows, int direction)
 {
     int64_t bucket = 1;
     while (bucket < rows) bucket <<= 1;
     std::ostringstream os;
-    os << "c2c.2:" << n << ":" << bucket << ":" << direction << ":" << device_name();
+    os << "c2c.3." << kernel_set() << ":" << n << ":" << bucket << ":" << direction << ":" << device_name();
     return os.str();
 }
 
@@ -287,9 +289,9 @@ std::vector<Tune> candidates(int64_t n)
             c.push_back(t);
         }
     } else {
-        // four-step splits n = a * b: the 8 most balanced ones (the default plan takes the most
-        // balanced pair of column leaves), each with three column-tile widths and the second stage on
-        // the rows-in / columns-out kernel or on the two-plane tile
+        // four-step splits n = a * b: the 8 most balanced ones beside the default plan's own (the first candidate:
+        // line alignment, passes, balance, then the stages' measured rates), each with three column-tile widths and
+        // the second stage on the rows-in / columns-out kernel or on the two-plane tile
         std::vector<std::pair<double, int64_t>> splits;
         for (int64_t a = 2; a <= 1024 && a < n; a++) {
             if (n % a || !find_instance(a)) continue;

@@ -1668,7 +1668,7 @@ std::string plan_describe(const Plan &p)
     std::ostringstream os;
     os << "{\"type\":" << p.fftType << ",\"direction\":" << p.direction << ",\"sizes\":[";
     for (size_t i = 0; i < p.sizes.size(); i++) os << (i ? "," : "") << p.sizes[i];
-    os << "],\"batch\":" << p.batch << ",\"dimType\":" << p.dimType << ",\"workspace\":" << p.ws_bytes;
+    os << "],\"batch\":" << p.batch << ",\"dimType\":" << p.dimType << ",\"workspace\":" << p.ws_bytes << ",\"kernels\":\"" << kernel_set() << "\"";
     os << ",\"stages\":[";
     for (size_t i = 0; i < p.stages.size(); i++) {
         const Stage &s = p.stages[i];

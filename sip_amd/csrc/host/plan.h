@@ -197,6 +197,8 @@ std::string plan_describe(const Plan &p);
 const StockhamInstance *find_instance(int64_t L);
 // Single-plane kernels of a role and length, or null.
 const RoleInstance *find_role(Role role, int64_t L);
+// Digest of the kernel sources that this library was built from: saved tuning results hold for them only.
+const char *kernel_set();
 // Measured GB/s of a length as first and second four-step stage (0, 0: not measured).
 std::pair<int, int> split_rates(int64_t L);
 // Split-precision MFMA instances (mode = PrecisionMode) and their DFT-matrix operand table.

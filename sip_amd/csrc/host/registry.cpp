@@ -80,6 +80,13 @@ const RoleInstance *find_role(Role role, int64_t L)
     return it == m.end() ? nullptr : it->second;
 }
 
+const char *kernel_set()
+{
+    return
+#include "kernel_set.inc"
+        ;
+}
+
 std::pair<int, int> split_rates(int64_t L)
 {
     static const std::map<int64_t, std::pair<int, int>> m = {

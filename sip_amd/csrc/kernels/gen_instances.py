@@ -11,6 +11,7 @@ OUTDIR/stockham_parts.inc). The output is a pure function of this file.
 """
 from __future__ import annotations
 
+import hashlib
 import os
 import sys
 
@@ -474,6 +475,23 @@ def write_istft(outdir):
     write_if_changed(os.path.join(outdir, "istft_parts.inc"), "\n".join(inc) + "\n")
 
 
+def kernel_set(outdir):
+    """Digest of every kernel source: the generated instances and the files beside this one."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    h = hashlib.sha256()
+    for d, ends in ((here, (".h", ".hip")), (outdir, (".hip", "_rates.inc"))):
+        for name in sorted(os.listdir(d)):
+            if name.endswith(ends):
+                with open(os.path.join(d, name), "rb") as fh:
+                    h.update(name.encode() + fh.read())
+    return h.hexdigest()[:8]
+
+
+def write_kernel_set(outdir):
+    text = ["// Generated by gen_instances.py (do not edit): digest of the kernel sources.", f'"{kernel_set(outdir)}"']
+    write_if_changed(os.path.join(outdir, "kernel_set.inc"), "\n".join(text) + "\n")
+
+
 def main():
     outdir = sys.argv[1]
     nparts = int(sys.argv[2])
@@ -515,6 +533,7 @@ def main():
     for k in range(nparts):
         inc.append(f"SIP_STOCKHAM_PART({k})")
     write_if_changed(os.path.join(outdir, "stockham_parts.inc"), "\n".join(inc) + "\n")
+    write_kernel_set(outdir)
     print(f"{len(inst)} leaf lengths in {nparts} parts")
 
 

@@ -319,3 +319,41 @@ def test_persistent_tuned_radix_orders(torch_cuda, tmp_path, monkeypatch):
         for a, b in zip(first, ys):
             assert torch.equal(a, b)
     bh.destroy()
+
+
+_TUNE_CHILD = """
+import json, sys, torch
+import sip_amd as S
+x = torch.zeros(256, 1024, dtype=torch.complex64, device="cuda")
+y = torch.empty_like(x)
+b = S.BatchHandle()
+assert b.make_plan([1024], [256], [x.data_ptr()], [y.data_ptr()], S.ASCEND_FFT_FORWARD, S.BATCH_AUTOTUNE) == 0
+print(json.dumps(b.describe()["group_list"][0]))
+b.destroy()
+"""
+
+
+def test_saved_tuning_of_other_kernels_is_ignored(torch_cuda, tmp_path):
+    """Entries of the tuning cache hold for the kernels they were timed with: one of an earlier library is not
+    taken, one of this library is (a child process each, the cache is read once per process)."""
+    import json
+    import os
+    import subprocess
+    import sys
+    torch = torch_cuda
+    arch = torch.cuda.get_device_properties(0).gcnArchName
+    cache = tmp_path / "tune.jsonl"
+    stale = "c2c.2:1024:256:%d:%s" % (FWD, arch)
+    cache.write_text('{"key":"%s","row_F":1,"split_lds":0,"xcd":0,"split_l1":0,"col_F":0,"rc":-1}\n' % stale)
+    env = dict(os.environ, SIP_FFT_TUNE_CACHE=str(cache), PYTHONPATH=os.path.dirname(S.HERE))
+
+    def child():
+        r = subprocess.run([sys.executable, "-c", _TUNE_CHILD], env=env, capture_output=True, text=True, timeout=100)
+        assert r.returncode == 0, r.stderr[-2000:]
+        return json.loads(r.stdout.strip().splitlines()[-1])
+
+    kernels = S.describe_dry([1024], S.ASCEND_FFT_C2C, FWD, 256)["kernels"]
+    assert child()["tuned_us"] > 0  # timed, not taken from the stale entry
+    keys = [json.loads(line)["key"] for line in cache.read_text().splitlines()]
+    assert keys == [stale, "c2c.3.%s:1024:256:%d:%s" % (kernels, FWD, arch)]
+    assert child()["tuned_us"] < 0  # taken from the entry of these kernels

@@ -133,3 +133,27 @@ def test_half_ulp_check_catches_a_misrounded_entry():
     bad[5] = np.complex64(np.nextafter(np.float32(t[5].real), np.float32(2)) + 1j * t[5].imag)
     with pytest.raises(AssertionError):
         assert_within_half_ulp(bad, re, im, "perturbed")
+
+
+def test_kernel_set_digest(tmp_path):
+    """The library names the kernels it was built from, and another shape makes another name (saved tuning
+    results hold for one name only)."""
+    import importlib.util
+    import os
+    import shutil
+    path = os.path.join(S.HERE, "csrc", "kernels", "gen_instances.py")
+    spec = importlib.util.spec_from_file_location("gen_instances_for_digest", path)
+    gen = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(gen)
+    built = os.path.join(S.HERE, "_gen")
+    if not os.path.isdir(built):
+        pytest.skip("the generated sources of the library are not here")
+    name = S.describe_dry([1024], S.ASCEND_FFT_C2C, FWD, 1)["kernels"]
+    assert name == gen.kernel_set(built)
+    other = tmp_path / "gen"
+    shutil.copytree(built, other)
+    part = other / "rows_part_0.hip"
+    text = part.read_text()
+    assert "ROLE_ROWS, 0, 0, 0," in text
+    part.write_text(text.replace("ROLE_ROWS, 0, 0, 0,", "ROLE_ROWS, 0, 2, 0,", 1))
+    assert gen.kernel_set(str(other)) != name
