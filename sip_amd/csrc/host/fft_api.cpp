@@ -60,13 +60,18 @@ int32_t finish_plan(Plan &p)
 {
     p.initialized = false;
     p.failed = false;
-    p.stages.clear();
+    auto clear = [&] {
+        p.stages.clear();
+        p.fusions.clear();
+        p.launches.clear();  // points into both
+    };
+    clear();
     try {
         sip::plan_build(p);
         sip::plan_materialize(p);
     } catch (...) {
         p.failed = true;
-        p.stages.clear();
+        clear();
         throw;
     }
     p.initialized = true;

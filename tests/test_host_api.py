@@ -373,3 +373,17 @@ def test_measured_radix_sequences_are_built():
     for n, seq in sorted(_seq_override().items()):
         st = dry([n], S.ASCEND_FFT_C2C, 256)["stages"][0]
         assert st["L"] == n and st["radices"] == list(seq), (n, st["radices"], seq)
+
+
+def test_failed_plan_keeps_nothing():
+    """A plan that could not be made (here: no GPU to make it on) describes no stages and no launches."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("needs a host without a GPU")
+    h = S.FftHandle()
+    try:
+        assert h.make_plan_1d(1009, S.ASCEND_FFT_C2C, S.ASCEND_FFT_FORWARD, 40) != S.ACL_SUCCESS
+        d = h.describe()
+        assert d["stages"] == [] and d["fused"] == []
+    finally:
+        h.destroy()
