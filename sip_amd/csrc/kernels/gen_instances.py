@@ -103,8 +103,6 @@ LEAF_SEQ = {
     25920: [16, 9, 9, 5, 4],  # 206 / 193
     30000: [10, 10, 10, 6, 5],  # 258 / 215
 }
-# The sequences these lengths run as contiguous rows: the row kernel's own where one was measured faster.
-SEQ_OVERRIDE = {n: ROW_SHAPES[n][1] if n in ROW_SHAPES else seq for n, seq in LEAF_SEQ.items()}
 # (1000 = 10 x 10 x 10 was faster in the four-step roles, 305 / 283 us, but its 100 threads per
 # transform halve the column tiles to 8 transforms, half-line HBM runs: 2D 1000^2 gained nothing.)
 

@@ -116,13 +116,15 @@ def _measured_lengths():
     spec = importlib.util.spec_from_file_location("gen_instances_for_test", path)
     mod = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(mod)
-    return sorted(mod.SEQ_OVERRIDE)
+    return sorted(mod.LEAF_SEQ)
 
 
 @pytest.mark.parametrize("n", _measured_lengths())
-def test_c2c_measured_radix_sequences(torch_cuda, n):
-    """Lengths whose radix sequence was chosen by measurement: forward against the oracle and the
-    round trip, at a batch that runs them as leaves (256 rows from 16384 up)."""
+def test_c2c_measured_radix_sequences(torch_cuda, monkeypatch, n):
+    """Lengths whose leaf's radix sequence was chosen by measurement: forward against the oracle and the
+    round trip, on the two-plane leaf (the row kernels have shapes of their own) and at a batch that runs
+    them as leaves (256 rows from 16384 up)."""
+    monkeypatch.setenv("SIP_FFT_SPLIT_LDS", "0")
     b = 256 if n > 16384 else max(2, min(64, (1 << 20) // n))
     x, y = _c2c_case(n, b, FWD, seed=8800 + n)
     back = c2c(y, [n], INV) / n
