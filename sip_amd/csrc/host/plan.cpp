@@ -146,15 +146,21 @@ static void four_step_tables(int64_t ntot, int sign, TableRef &lo, TableRef &hi)
 }
 
 // FP64 forward FFT of a 2,3,5-smooth length (host; plan-time table generation only): Stockham
-// passes of radix 4, 2, 3 and 5 with the roots evaluated once.
+// passes of radix 4, 2, 3 and 5 with the roots evaluated once, a quarter or half of them where the others are
+// those times -i and -1 (the long-double sines and cosines are most of the time of a long table).
 static void fft_smooth_f64(std::vector<double> &re, std::vector<double> &im)
 {
     const size_t n = re.size();
     std::vector<double> wr(n), wi(n), tr(n), ti(n);
-    for (size_t m = 0; m < n; m++) {
+    const size_t own = n % 4 == 0 ? n / 4 : n % 2 == 0 ? n / 2 : n;
+    for (size_t m = 0; m < own; m++) {
         const long double a = -6.283185307179586476925286766559005768L * (long double)m / (long double)n;
         wr[m] = (double)cosl(a);
         wi[m] = (double)sinl(a);
+    }
+    for (size_t m = own; m < n; m++) {
+        wr[m] = n % 4 == 0 ? wi[m - own] : -wr[m - own];
+        wi[m] = n % 4 == 0 ? -wr[m - own] : -wi[m - own];
     }
     size_t ns = 1;
     while (ns < n) {
