@@ -25,30 +25,16 @@
 
 namespace sip {
 
-template <int R, int... Rest>
-struct LastRadix {
-    static constexpr int value = LastRadix<Rest...>::value;
-};
-template <int R>
-struct LastRadix<R> {
-    static constexpr int value = R;
-};
-
 template <int W, int L, int T, int... Rs>
 __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(W))) void istft_kernel(const IstftArgs a)
 {
     extern __shared__ float pl[];
     constexpr int R0 = first_of<Rs...>(), NBF0 = L / R0, NB0 = (NBF0 + T - 1) / T;
     constexpr bool EXACT0 = (NBF0 % T) == 0;
-    constexpr int RL = LastRadix<Rs...>::value, NBFL = L / RL, NBL = (NBFL + T - 1) / T;
+    constexpr int RL = last_of<Rs...>(), NBFL = L / RL, NBL = (NBFL + T - 1) / T;
     constexpr bool EXACTL = (NBFL % T) == 0;
     const int F = a.F, tid = threadIdx.x, nthreads = blockDim.x;
-    // XCD-contiguous order: workgroups go round robin to the 8 XCDs, each takes a contiguous range
-    int64_t tile = blockIdx.x;
-    {
-        const int64_t nt = gridDim.x, q = nt / 8, rem = nt % 8, x = tile % 8;
-        tile = x * q + (x < rem ? x : rem) + tile / 8;
-    }
+    const int64_t tile = xcd_tile();
     const uint32_t c = fdiv((uint32_t)tile, a.div_tiles);
     const int64_t k = tile - (int64_t)c * a.tiles;
     const int64_t t0 = k * a.keep - a.halo;  // first frame of the tile

@@ -58,15 +58,6 @@ __global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(W))) void 
                                           PlanesIo{static_cast<float *>(a.out) + ob, a.out_im + ob});
 }
 
-template <int R, int... Rest>
-constexpr int last_radix()
-{
-    if constexpr (sizeof...(Rest) == 0)
-        return R;
-    else
-        return last_radix<Rest...>();
-}
-
 // Rows in line order: element i = tid + u (F T) of the workgroup's F L contiguous elements. The exchange
 // between line order and the passes' order goes through the plane in two halves on both sides. Rows of a
 // tile are contiguous (the host checks that a row starts where the one before ends).
@@ -74,7 +65,7 @@ template <int L, int T, int... Rs>
 __global__ __launch_bounds__(1024) void planes_small_kernel(const StockhamArgs a)
 {
     extern __shared__ float pl[];
-    constexpr int R0 = first_of<Rs...>(), RL = last_radix<Rs...>();
+    constexpr int R0 = first_of<Rs...>(), RL = last_of<Rs...>();
     constexpr int NBF0 = L / R0, NB0 = (NBF0 + T - 1) / T, NBFL = L / RL, NBL = (NBFL + T - 1) / T;
     constexpr int NG = (L + T - 1) / T;
     const int F = a.F, tid = threadIdx.x, nt = blockDim.x;

@@ -130,15 +130,6 @@ struct Tile2d<X, TX, Y, TY, S, Radices<RX...>, Radices<RY...>> {
     }
 };
 
-template <int A, int... Rest>
-constexpr int last_of()
-{
-    if constexpr (sizeof...(Rest) == 0)
-        return A;
-    else
-        return last_of<Rest...>();
-}
-
 // The same slice with one LDS plane (a 128 x 128 slice takes 70 KiB, so two workgroups share a CU); every exchange
 // moves the real parts through it, then the imaginary parts. The first row pass reads HBM (TY threads per
 // row, runs of TY values) and the last column pass writes HBM with lanes along y, so a slice goes through

@@ -54,6 +54,15 @@ constexpr int first_of()
     return A;
 }
 
+template <int A, int... Rest>
+constexpr int last_of()
+{
+    if constexpr (sizeof...(Rest) == 0)
+        return A;
+    else
+        return last_of<Rest...>();
+}
+
 // Padded LDS index of element base + r * STRIDE for a compile-time STRIDE. When the padding of
 // the r-dependent part is a compile-time constant the result is pad(base) + const(r), so a
 // butterfly's R accesses share one address and differ only in the instruction's offset field.
@@ -599,17 +608,18 @@ __device__ __forceinline__ void split_rows_c2r(const StockhamArgs &a, float *pl,
                                          RowIo{nullptr, static_cast<float2 *>(a.out) + ob});
 }
 
-// Tile of this workgroup; with xcd_remap the round-robin dispatch of consecutive workgroups to the
-// 8 XCDs is undone so that each XCD streams through one contiguous range of tiles.
+// Tile of this workgroup in XCD order: the round-robin dispatch of consecutive workgroups to the 8 XCDs is
+// undone so that each XCD streams through one contiguous range of tiles.
+__device__ __forceinline__ int64_t xcd_tile()
+{
+    const int64_t tile = blockIdx.x, ntiles = gridDim.x, q = ntiles / 8, rem = ntiles % 8;
+    const int64_t x = tile % 8, sl = tile / 8;
+    return x * q + (x < rem ? x : rem) + sl;
+}
+
 __device__ __forceinline__ int64_t tile_index(const StockhamArgs &a)
 {
-    int64_t tile = blockIdx.x;
-    if (a.xcd_remap) {
-        const int64_t ntiles = gridDim.x, q = ntiles / 8, rem = ntiles % 8;
-        const int64_t x = tile % 8, sl = tile / 8;
-        tile = x * q + (x < rem ? x : rem) + sl;
-    }
-    return tile;
+    return a.xcd_remap ? xcd_tile() : (int64_t)blockIdx.x;
 }
 
 // Strided transform of a column tile: element j at in[j * es_in] / out[j * es_out], with the
