@@ -1429,14 +1429,16 @@ void plan_materialize_external(Plan &p, const std::vector<const int64_t *> &dev_
 // half of that cache: two such tiles per CU read more than the intermediate can share the cache with. us on three
 // buffer sets in turn / on one set over and over / on one set that the kernel before writes (both kernels), cached ->
 // nontemporal: 1048576 x 8 70.9 -> 53.3 / 52.9 -> 54.5 / 61.3 -> 61.2, 1024000 x 8 71.8 -> 63.9 / 62.8 -> 63.4 / 72.3 ->
-// 71.2. Shorter first stages and rows keep cached loads: what they gain on cold inputs (65536 x 128 54.4 -> 50.6, 1024^2
-// x 16 101.6 -> 95.0) they lose on the inputs of a program that has just written or read them (46.7 -> 51.2, 90.9 ->
-// 95.5), half lines more (40000 x 220 after a pass over its input 71.8 -> 86.1).
+// 71.2. Shorter first stages in whole lines do so beyond 288 MiB (inputs of 96 MiB): 65536 x 224 89.3 -> 84.2 / 89.2 ->
+// 85.3 / 117.6 -> 114.7, 432000 x 46 167.8 -> 144.1 / 167.8 -> 146.0 / 205.5 -> 195.3, 131072 x 198 178 -> 159 / 178 ->
+// 159 / 245 -> 213; at 64 MiB what they gain on cold inputs (65536 x 128 54.4 -> 50.6) they lose on the inputs of a
+// program that has just written or read them (46.7 -> 51.2). Rows and half lines keep cached loads at every size: 1024^2
+// x 16 gains 101.6 -> 95.0 and loses 90.9 -> 95.5, x 20 119.8 -> 140.1; 40000 x 220 after a pass over its input 71.8 -> 86.1.
 void plan_mark_streaming(Plan &p)
 {
     const bool on_out = env_flag("SIP_FFT_NT_OUT", true), on_in = env_flag("SIP_FFT_NT_IN", true);
     constexpr int64_t kNtInBytes = int64_t(512) << 20;
-    constexpr int64_t kNtInFootprint = int64_t(128) << 20;
+    constexpr int64_t kNtInFootprint = int64_t(128) << 20, kNtInBeyond = int64_t(288) << 20;
     const std::vector<Stage *> run = plan_launches(p);
     const bool gathered = !p.row_tables.empty() || !p.external_tables.empty();
     int64_t footprint = 0;  // bytes read by the first launch and written outside in-place steps
@@ -1486,7 +1488,7 @@ void plan_mark_streaming(Plan &p)
         s.sa.nt_out = (on_out && !read_later && aligned_out) ? 1 : 0;
         const int64_t in_bytes = s.sa.nfft * (int64_t)s.sa.in_len * 8;
         const bool cold = i == 0 && run.size() > 1 && s.in.kind == BUF_IN && !gathered && footprint > kNtInFootprint &&
-                          cols_in && s.sa.tin.es % 16 == 0 && s.sa.in_len >= 1000;
+                          cols_in && s.sa.tin.es % 16 == 0 && (s.sa.in_len >= 1000 || footprint > kNtInBeyond);
         s.sa.nt_in = (on_in && s.sa.io_mode == IO_C2C && (in_bytes >= kNtInBytes || cold) && aligned_in) ? 1 : 0;
     }
 }

@@ -102,7 +102,7 @@ def test_column_shapes_with_twiddle(torch_cuda, monkeypatch, n):
 
 
 def test_streaming_input_of_several_launches(torch_cuda):
-    """A plan of several launches that touches more than 128 MiB loads its input nontemporally."""
+    """A first stage of long whole-line columns in a plan that touches more than 128 MiB loads its input nontemporally."""
     h = make([1 << 20], S.ASCEND_FFT_C2C, FWD, 8)
     assert [s["nt_in"] for s in h.describe()["stages"]] == [1, 0]
     h.destroy()

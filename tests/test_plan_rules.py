@@ -100,11 +100,12 @@ def test_real_rows_on_one_or_two_planes(n, start):
         assert at == ([0, 0, 1] if start else [1, 1, 1])
 
 
-@pytest.mark.parametrize("dims,b,nt", [([1 << 20], 8, 1), ([1 << 20], 5, 0), ([1024000], 8, 1), ([65536], 128, 0), ([65536], 256, 0),
+@pytest.mark.parametrize("dims,b,nt", [([1 << 20], 8, 1), ([1 << 20], 5, 0), ([1024000], 8, 1), ([65536], 128, 0), ([65536], 192, 0),
+                                       ([65536], 193, 1), ([432000], 40, 1), ([40000], 400, 0),
                                        ([262144], 32, 0), ([40000], 220, 0), ([1000000], 8, 0), ([524288], 16, 0),
                                        ([1024, 1024], 16, 0), ([720, 1280], 16, 0), ([256, 256, 256], 2, 0)])
 def test_streaming_inputs(dims, b, nt):
-    """Below 512 MiB only long first-stage columns in whole lines pass the last-level cache."""
+    """Below 512 MiB only first-stage columns in whole lines pass the last-level cache, short ones from 96 MiB of input."""
     assert S.describe_dry(dims, C2C, FWD, b)["stages"][0]["nt_in"] == nt
 
 
