@@ -569,12 +569,13 @@ struct Builder {
             // A tile of half a wave or less takes a whole one: one thread per column 64 wide (16 / 64 wide: 20 x
             // 4096 3.28 / 2.89 us, 20 x 262144 23.1 / 15.1, 3 x 262144 6.0 / 3.5), two 32 wide (16 / 32: 24 x 4096
             // 3.96 / 3.60, 40 x 131072 19.7 / 14.9). Three keep 16 (16 / 32: 36 x 4096 3.63 / 3.87, 45 x 16384 5.07 /
-            // 5.34, 60 x 131072 34.1 / 32.9), and so do the stages of a split, whose second launch finds in each
-            // XCD's cache what the first left there only where both cut the columns alike (2D 1080 x 1024 x 1 as
-            // 20 x 54, 64 and 16 wide 24.7 us, both 16 wide 22.5).
+            // 5.34, 60 x 131072 34.1 / 32.9), and so do the stages of a split in launch order, whose second launch finds
+            // in each XCD's cache what the first left there only where both cut the columns alike (2D 1080 x 1024 x 1 as
+            // 20 x 54, 64 and 16 wide 24.7 us, both 16 wide 22.5). In XCD order (split lines) each XCD keeps its range of
+            // columns at any width: 2D 1500 x 162 x 4 as 20 x 75, 64 and 16 wide 22.1 us, both 16 wide 24.2.
             const bool pow2 = (L & (L - 1)) == 0;
             if (want <= 0 && role) want = role->F;
-            F = want > 0 ? want : pow2 ? std::min(64, std::max(16, (512 / T) & ~15)) : T >= 3 || tw4_ntot ? 16 : T == 2 ? 32 : 64;
+            F = want > 0 ? want : pow2 ? std::min(64, std::max(16, (512 / T) & ~15)) : T >= 3 || (tw4_ntot && a.tin.es % 16 == 0) ? 16 : T == 2 ? 32 : 64;
             if (F >= 16) F &= ~15;
             while (F > 1 && ((size_t)F * per > 160 * 1024 || F * T > 1024)) F /= 2;
             // Few tiles: 8 wide where 16 would leave half of the CUs without one (out of place: in place, half

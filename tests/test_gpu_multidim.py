@@ -38,7 +38,7 @@ def test_c3_3d_128cube_b4_tones(torch_cuda):
 @pytest.mark.parametrize("dims,batch", [((64, 64), 2), ((100, 200), 3), ((2048, 3000), 1), ((7, 13), 5),
                                         ((4096, 33), 1), ((1, 128), 4), ((128, 1), 4), ((17, 31), 2),
                                         ((32, 48, 20), 2), ((8, 8, 8), 7), ((5, 1024, 3), 1), ((1, 1, 64), 2),
-                                        ((30, 997, 2), 1)])
+                                        ((30, 997, 2), 1), ((1500, 162), 4), ((1500, 33), 1), ((1200, 90), 2)])
 def test_c2c_nd(torch_cuda, dims, batch):
     x = oracle.uniform_complex((batch,) + dims, seed=sum(dims) + batch)
     tol = 5e-6 if any(d in (17, 31, 997) for d in dims) else TOL

@@ -50,10 +50,12 @@ def test_column_tile_widths(n, width):
 
 
 def test_split_stages_cut_columns_alike():
-    """A split axis of few-thread factors keeps one tile width in both launches."""
+    """A split axis of few-thread factors keeps one tile width in both launches, but in XCD order."""
     for n in (1080, 1200):
         st = S.describe_dry([n, 1024], C2C, FWD, 1)["stages"][1:]
         assert len(st) == 2 and [s["F"] for s in st] == [16, 16]
+    st = S.describe_dry([1500, 162], C2C, FWD, 4)["stages"][1:]
+    assert [s["F"] for s in st] == [64, 16] and [s["xcd_remap"] for s in st] == [1, 1]
 
 
 @pytest.mark.parametrize("n,rows", [(12150, 257), (12960, 257), (14580, 257), (15000, 257), (16000, 320)])
